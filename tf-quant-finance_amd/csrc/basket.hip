@@ -44,6 +44,8 @@ basket_kernel(const float* __restrict__ prm, int n_steps, float t, float r,
   for (int e = threadIdx.x; e < (kBlockK / kWave) * 2 * NS; e += kBlockK)
     (&red[0][0])[e] = 0.0;
   __syncthreads();
+  PhiloxKeys<true> keys;
+  keys.init(k0, k1);
   // rounds are uniform over the block; lanes past n_paths compute a valid
   // path and contribute zero
   for (int64_t p0 = (int64_t)blockIdx.x * kBlockK; p0 < n_paths;
@@ -61,7 +63,7 @@ basket_kernel(const float* __restrict__ prm, int n_steps, float t, float r,
         const int j = st * D + i;  // D % 4 == 0 keeps j % 4 == 0
         const u32x4 w = philox4x32_10(
             u32x4{(uint32_t)p, (uint32_t)(j >> 2), stream, (uint32_t)(p >> 32)},
-            k0, k1);
+            keys);
         float z0, z1, z2, z3;
         box_muller(w.x, w.y, z0, z1);
         box_muller(w.z, w.w, z2, z3);

@@ -34,8 +34,8 @@ constexpr int kSeg = 16;  // steps per checkpoint segment
 
 __device__ __forceinline__ void normals4(uint32_t p_lo, uint32_t p_hi,
                                          uint32_t blk, uint32_t stream,
-                                         uint32_t k0, uint32_t k1, float* z) {
-  const u32x4 w = philox4x32_10(u32x4{p_lo, blk, stream, p_hi}, k0, k1);
+                                         const PhiloxKeys<true>& keys, float* z) {
+  const u32x4 w = philox4x32_10(u32x4{p_lo, blk, stream, p_hi}, keys);
   box_muller(w.x, w.y, z[0], z[1]);
   box_muller(w.z, w.w, z[2], z[3]);
 }
@@ -70,8 +70,7 @@ __device__ __forceinline__ void load_contract(const tqf_contract* __restrict__ c
 
 // One GBM path: price and (delta, vega, rho).
 __device__ __forceinline__ void gbm_path(const Contract& c, int64_t p,
-                                         uint32_t stream, uint32_t k0,
-                                         uint32_t k1, float* g) {
+                                         uint32_t stream, const PhiloxKeys<true>& keys, float* g) {
   const float dt = c.t / (float)c.n_steps;
   const float sdt = sqrtf(dt);
   const float drift = (c.r - 0.5f * c.sigma * c.sigma) * dt;
@@ -80,8 +79,7 @@ __device__ __forceinline__ void gbm_path(const Contract& c, int64_t p,
   // four steps per Philox block (block i / 4 serves steps i .. i + 3)
   int i = 0;
   for (; i + 4 <= c.n_steps; i += 4) {
-    normals4((uint32_t)p, (uint32_t)(p >> 32), (uint32_t)(i >> 2), stream, k0,
-             k1, z);
+    normals4((uint32_t)p, (uint32_t)(p >> 32), (uint32_t)(i >> 2), stream, keys, z);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float dw = z[u] * sdt;
@@ -90,8 +88,7 @@ __device__ __forceinline__ void gbm_path(const Contract& c, int64_t p,
     }
   }
   if (i < c.n_steps) {
-    normals4((uint32_t)p, (uint32_t)(p >> 32), (uint32_t)(i >> 2), stream, k0,
-             k1, z);
+    normals4((uint32_t)p, (uint32_t)(p >> 32), (uint32_t)(i >> 2), stream, keys, z);
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       if (i + u < c.n_steps) {
@@ -131,7 +128,8 @@ __device__ __forceinline__ void heston_step(const Contract& c, float xr,
 // One Heston path with the checkpointed reverse sweep.  ck: this thread's
 // checkpoint column (stride `cstride` floats between segments).
 __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
-                            uint32_t k0, uint32_t k1, float* __restrict__ ck,
+                            const PhiloxKeys<true>& keys,
+                            float* __restrict__ ck,
                             int64_t cstride, float* g) {
   const int n = c.n_steps;
   const float dt = c.t / (float)n;
@@ -148,7 +146,7 @@ __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
       ck[(int64_t)(i / kSeg) * 2 * cstride + cstride] = v;
     }
     if ((i & 1) == 0)
-      normals4(plo, phi, (uint32_t)(i >> 1), stream, k0, k1, z);
+      normals4(plo, phi, (uint32_t)(i >> 1), stream, keys, z);
     const float z0 = (i & 1) ? z[2] : z[0];
     const float z1 = (i & 1) ? z[3] : z[1];
     heston_step(c, xr, xs, dt, sdt, z0, z1, x, v);
@@ -171,7 +169,7 @@ __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
       const int i = i0 + u;
       if (i < n) {
         if ((u & 1) == 0)
-          normals4(plo, phi, (uint32_t)(i >> 1), stream, k0, k1, z);
+          normals4(plo, phi, (uint32_t)(i >> 1), stream, keys, z);
         z0s[u] = (u & 1) ? z[2] : z[0];
         z1s[u] = (u & 1) ? z[3] : z[1];
         xs_[u] = cx;
@@ -222,8 +220,7 @@ __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
 //   x'  <- x' - dt/2 v+' + sqrt(v+)' dw0
 //   v'  <- v' - dt kappa v+' + sqrt(v+)' (xi rho dw0 + xi s dw1) + dv'/dp
 __device__ void heston_path_tangent(const Contract& c, int64_t p,
-                                    uint32_t stream, uint32_t k0,
-                                    uint32_t k1, float* g) {
+                                    uint32_t stream, const PhiloxKeys<true>& keys, float* g) {
   const int n = c.n_steps;
   const float dt = c.t / (float)n;
   const float sdt = sqrtf(dt);
@@ -239,7 +236,7 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
   float z[4];
   for (int i = 0; i < n; ++i) {
     if ((i & 1) == 0)
-      normals4(plo, phi, (uint32_t)(i >> 1), stream, k0, k1, z);
+      normals4(plo, phi, (uint32_t)(i >> 1), stream, keys, z);
     const float z0 = (i & 1) ? z[2] : z[0];
     const float z1 = (i & 1) ? z[3] : z[1];
     const bool pos = v > 0.f;
@@ -299,6 +296,8 @@ batch_kernel(const tqf_contract* __restrict__ contracts,
   __shared__ double red[kBlockB / kWave][2 * kStats];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float* ck = ckpt + (int64_t)blockIdx.x * ckpt_per_block + threadIdx.x;
+  PhiloxKeys<true> keys;
+  keys.init(k0, k1);
   int next = blockIdx.x;
   for (;;) {
     if (use_counter) {
@@ -319,15 +318,15 @@ batch_kernel(const tqf_contract* __restrict__ contracts,
          p += kBlockB) {
       float g[kStats];
       if (c.kind == TQF_CONTRACT_GBM)
-        gbm_path(c, p, c.stream, k0, k1, g);
+        gbm_path(c, p, c.stream, keys, g);
       else if (!kAdjoint || c.greeks_mode == TQF_GREEKS_TANGENT ||
                (c.n_steps + kSeg - 1) / kSeg > max_seg)
         // a contract with more steps than the checkpoint workspace holds
         // (n_steps > max_steps) takes the forward tangents, the same
         // estimator, rather than write past its checkpoint column
-        heston_path_tangent(c, p, c.stream, k0, k1, g);
+        heston_path_tangent(c, p, c.stream, keys, g);
       else
-        heston_path(c, p, c.stream, k0, k1, ck, kBlockB, g);
+        heston_path(c, p, c.stream, keys, ck, kBlockB, g);
 #pragma unroll
       for (int q = 0; q < kStats; ++q) {
         acc[q] += g[q];

@@ -135,8 +135,11 @@ struct Normals {
       RNG == TQF_RNG_SOBOL || RNG == TQF_RNG_SOBOL_SHIFTED;
   static constexpr bool kIcdf =
       RNG == TQF_RNG_SOBOL_SHIFTED && sizeof(R) == sizeof(float);
+  static constexpr bool kPhilox =
+      RNG == TQF_RNG_PHILOX || RNG == TQF_RNG_PHILOX_ANTITHETIC;
   R c0, c1, c2, c3;  // Philox cache
   uint32_t ctr0, ctr3;
+  PhiloxKeys<sizeof(R) == sizeof(float)> keys;
   R sign;
   int64_t p;
   uint32_t lo_idx, hi_sel;
@@ -171,6 +174,7 @@ struct Normals {
     }
     ctr0 = (uint32_t)p;
     ctr3 = (uint32_t)(p >> 32);
+    if constexpr (kPhilox) keys.init(a.k0, a.k1);
     if (kSobol) {
       const uint64_t idx = (uint64_t)(a.sfirst + path);
       const uint64_t hi0 =
@@ -258,7 +262,7 @@ struct Normals {
       const int r = j & 3;
       if (r == 0) {
         const u32x4 w = philox4x32_10(
-            u32x4{ctr0, (uint32_t)(j >> 2), a.stream_id, ctr3}, a.k0, a.k1);
+            u32x4{ctr0, (uint32_t)(j >> 2), a.stream_id, ctr3}, keys);
         box_muller(w.x, w.y, c0, c1);
         box_muller(w.z, w.w, c2, c3);
       }

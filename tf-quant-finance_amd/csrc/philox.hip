@@ -21,9 +21,11 @@ philox_normals_kernel(uint32_t k0, uint32_t k1, uint32_t stream_id,
     src = p - n_paths / 2;
     sign = (R)-1;
   }
+  PhiloxKeys<false> keys;  // one block per thread: nothing to amortise
+  keys.init(k0, k1);
   const u32x4 w = philox4x32_10(
-      u32x4{(uint32_t)src, (uint32_t)b, stream_id, (uint32_t)(src >> 32)}, k0,
-      k1);
+      u32x4{(uint32_t)src, (uint32_t)b, stream_id, (uint32_t)(src >> 32)},
+      keys);
   R z[4];
   box_muller(w.x, w.y, z[0], z[1]);
   box_muller(w.z, w.w, z[2], z[3]);
