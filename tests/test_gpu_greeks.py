@@ -420,3 +420,54 @@ def test_batch_table_sample_price_and_greeks_vs_oracle(greeks):
       scale = max(abs(want[q]), 1e-2 * abs(price), 1e-6)
       assert abs(got - want[q]) <= 2e-3 * scale + 0.1 * want_se[q], (
           c['kind'], name, got, want[q], want_se[q])
+
+
+@pytest.mark.parametrize('greeks', ['tangent', 'adjoint'])
+def test_batch_short_contracts_and_item_counts_vs_oracle(greeks):
+  # the remainders of the step loops (four GBM steps, two Heston steps per
+  # Philox block) and of the per-contract sum (16 rows at a time: contracts
+  # of 1, 16, 17 and 33 items), against the float64 oracle on the same draws.
+  # Bound: a path's terms carry up to 4 roundings (6e-8 each) per step and
+  # about 10 from the normals and the payoff, under 40 x 6e-8 = 2.4e-6 of
+  # the term at 7 steps; sqrt(v+) turns a relative error e of v into e / 2
+  # and its reciprocal's derivative up to 3 e / 2, hence 4e-6, taken at
+  # 1e-5.  The terms of a Greek have both signs, so the mean's error is
+  # measured by their root mean square, not by the mean
+  cs = []
+  for i, (n, m) in enumerate([(1, 64), (2, 1024), (3, 1030), (4, 2112),
+                              (5, 64), (7, 1087)]):
+    cs.append(_gbm(2 * i, steps=n, paths=m))
+    # total noise of v about 0.2 sqrt(0.09 0.1) = 0.019: no path comes near
+    # v = 0, where the bound would not hold
+    cs.append(_heston(2 * i + 1, steps=n, paths=m, t=0.1, v0=0.09, xi=0.2,
+                      theta=0.09))
+  for i, c in enumerate(cs):
+    c['stream_id'] = i
+  plan = batch_lib.BatchPlan(cs, tile=64, seed=9, greeks=greeks)
+  plan.launch()
+  for c, r in zip(cs, plan.results()):
+    n, m = c['n_steps'], c['n_paths']
+    print(c['kind'], n, m, flush=True)
+    if c['kind'] == batch_lib.KIND_GBM:
+      z = orng.normals(m, n, 9, stream=c['stream_id'],
+                       dtype=np.float32).astype(np.float64)
+      w = np.sqrt(c['maturity'] / n) * z.sum(1)
+      s = c['s0'] * np.exp((c['rate'] - 0.5 * c['sigma']**2) * c['maturity'] +
+                           c['sigma'] * w)
+      disc = np.exp(-c['rate'] * c['maturity'])
+      sb = disc * np.where(s > c['strike'], s, 0)
+      pay = disc * np.maximum(s - c['strike'], 0)
+      want = [pay, sb / c['s0'], sb * (w - c['sigma'] * c['maturity']),
+              c['maturity'] * (sb - pay)]
+      rms = [np.sqrt(np.mean(np.square(g))) for g in want]
+      want = [g.mean() for g in want]
+    else:
+      z = orng.normals(m, 2 * n, 9, stream=c['stream_id'],
+                       dtype=np.float32).astype(np.float64).reshape(m, n, 2)
+      want, se = oheston.ft_euler_call_greeks(
+          np.log(c['s0']), c['v0'], c['kappa'], c['theta'], c['xi'], c['rho'],
+          c['rate'], c['strike'], np.linspace(0.0, c['maturity'], n + 1), z)
+      rms = np.sqrt(want**2 + m * se**2)
+    for q, name in enumerate(batch_lib.GREEK_NAMES[c['kind']]):
+      assert abs(r[name][0] - want[q]) <= 1e-5 * rms[q], (c['kind'], n, m,
+                                                         name)
