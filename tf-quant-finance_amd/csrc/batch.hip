@@ -119,7 +119,7 @@ __device__ __forceinline__ void gbm_path(const Contract& c, int64_t p,
 struct HestonConst {
   float sdt, sdt_lo;      // sqrt(dt)
   float mdt2;             // -dt / 2
-  float mdtk, dtkth;      // -dt kappa, dt kappa theta
+  float mdtk, theta;      // -dt kappa
   float xi, rho, s1r;
 };
 
@@ -130,7 +130,7 @@ __device__ __forceinline__ HestonConst heston_const(const Contract& c) {
   k.sdt_lo = (float)(sdt - (double)k.sdt);
   k.mdt2 = (float)(-0.5 * dt);
   k.mdtk = (float)(-dt * c.kappa);
-  k.dtkth = (float)(dt * c.kappa * c.theta);
+  k.theta = c.theta;
   k.xi = c.xi;
   k.rho = c.rho;
   k.s1r = (float)sqrt(1.0 - (double)c.rho * c.rho);
@@ -148,7 +148,7 @@ __device__ __forceinline__ void heston_step(const HestonConst& k, float vp,
                                             float sq, float dw0, float cu,
                                             float& x, float& v) {
   x = fma_r(sq, dw0, fma_r(vp, k.mdt2, x));
-  v += fma_r(k.xi * sq, cu, fma_r(vp, k.mdtk, k.dtkth));
+  v += fma_r(k.xi * sq, cu, k.mdtk * (vp - k.theta));
 }
 
 // Discounted payoff and dP/d ln S of the final state.
@@ -253,10 +253,10 @@ __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
 // with h = 1 / (2 sqrt v) and cu = rho dw0 + s dw1.  A and B are the same
 // for the five tangents, so each costs two FMAs (a select, a product and
 // four FMAs when the factors are applied one by one).  Bound by VALU issue:
-// 68 instructions and 230 cycles a step and wave, of which half a Philox
+// 69 instructions and 233 cycles a step and wave, of which half a Philox
 // block is 66 and the Box-Muller pair 62; five waves per SIMD (the launch
 // bound keeps it at 96 registers).  A book of 256 contracts (8.3e9 GBM and
-// 8.3e9 Heston path-steps) takes 4.36 ms, 5.68 ms before.
+// 8.3e9 Heston path-steps) takes 4.40 ms, 5.68 ms before.
 __device__ void heston_path_tangent(const Contract& c, int64_t p,
                                     uint32_t stream,
                                     const PhiloxKeys<true>& keys, float* g) {
@@ -264,7 +264,7 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
   const HestonConst k = heston_const(c);
   const double dt = (double)c.t / n;
   const float drho_s = -c.rho / k.s1r;  // d sqrt(1-rho^2) / d rho
-  const float mdt = (float)-dt, dtth = (float)(dt * c.theta);
+  const float mdt = (float)-dt;
   const float b0 = (float)(1.0 - dt * c.kappa);
   const uint32_t plo = (uint32_t)p, phi = (uint32_t)(p >> 32);
   float x = 0.f, v = c.v0;
@@ -285,7 +285,7 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
 #pragma unroll
     for (int q = 0; q < 5; ++q) tx[q] = fma_r(a, tv[q], tx[q]);
     tv[0] *= b;
-    tv[1] = fma_r(b, tv[1], fma_r(vp, mdt, dtth));               // kappa
+    tv[1] = fma_r(mdt, vp - k.theta, b * tv[1]);                 // kappa
     tv[2] = fma_r(b, tv[2], -k.mdtk);                            // theta
     tv[3] = fma_r(b, tv[3], sq * cu);                            // xi
     tv[4] = fma_r(b, tv[4], (k.xi * sq) * fma_r(drho_s, dw1, dw0));  // rho
