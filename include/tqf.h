@@ -389,6 +389,36 @@ int tqf_lsm_price(const tqf_lsm* lsm, const int32_t* ex_idx, int32_t n_ex,
                   const double* df, void* workspace, double* cash,
                   double* vals, double* result, int32_t* ranks, void* stream);
 
+/* One payoff of tqf_lsm_price_shared. */
+typedef struct tqf_lsm_item {
+  int32_t payoff;           /* TQF_PAYOFF_*                                  */
+  int32_t pad0;
+  double strike;
+  const double* payoff_table;  /* TQF_PAYOFF_TABLE: as tqf_lsm               */
+  const double* df;         /* host [n_ex + 1] padded discount factors (the
+                               lsm's path_discounts replace them when set)   */
+  const double* log_shift;  /* host [n_ex] or NULL.  With basis_log 2: the
+                               log price at exercise date e is log_shift[e]
+                               + log_scale * stored value                    */
+  double log_scale;
+} tqf_lsm_item;
+
+/* Device.  tqf_lsm_price for n_items (1..16) payoffs on the same one-asset
+ * paths (lsm->dim = 1, degree 0..4; lsm's payoff, strike, payoff_table,
+ * n_basis and exponents are not read): basis_mask bit m says that the
+ * monomial c^m is in the basis.  One launch per exercise date for all of
+ * them, no host synchronisation and no host copy.  values
+ * [n_items][n_paths] (device) receives each path's value at the first
+ * exercise date, before the final discount; results [n_items][2]; ranks
+ * (optional) [n_items][max(n_ex - 1, 1)]. */
+int64_t tqf_lsm_shared_workspace_size(int64_t n_paths, int32_t n_items,
+                                      int32_t n_ex);
+int tqf_lsm_price_shared(const tqf_lsm* lsm, const tqf_lsm_item* items,
+                         int32_t n_items, int32_t basis_mask,
+                         const int32_t* ex_idx, int32_t n_ex, void* workspace,
+                         double* values, double* results, int32_t* ranks,
+                         void* stream);
+
 /* Per-date building blocks of the same backward induction, for callers that
  * supply their own continuation estimate (the MLP model below):
  *   tqf_lsm_terminal     cash = payoff at t_idx, vals = 0

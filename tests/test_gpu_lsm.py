@@ -430,3 +430,68 @@ def test_one_asset_chain_every_degree_matches_oracle(degree):
       olsm.make_polynomial_basis(degree, True), discount_factors=dfs,
       num_calibration_samples=n // 3)[0]
   np.testing.assert_allclose(float(_np(got)[0]), want, rtol=2e-6)
+
+
+@pytest.mark.parametrize('n', [2, 255, 1024, 1025, 4097])
+def test_shared_paths_batch_equals_single_items_and_explicit_paths(n):
+  # price_shared: 17 payoffs (two launches' worth) on one set of paths, at
+  # path counts around a round (1,024) and a workgroup.  Each payoff equals
+  # itself priced alone bit for bit (the sums do not depend on the batch),
+  # and the affine map of the stored values equals explicit log-price paths:
+  # the standardised basis sees rounding only, 1e-16 relative amplified by
+  # the 3 x 3 solve's condition number (below 1e3), hence 1e-12
+  print('shared paths', n, flush=True)
+  g = torch.Generator(device='cuda').manual_seed(n)
+  steps = 6
+  w = torch.randn((steps, n), dtype=torch.float64, device='cuda',
+                  generator=g).cumsum(0) * 0.4
+  dev = w.device
+  t = np.arange(1, steps + 1) / steps
+  items, vols = [], np.linspace(0.1, 0.5, 17)
+  for i, vol in enumerate(vols):
+    items.append({'payoff': (lsm.PAYOFF_BASKET_PUT if i % 2
+                             else lsm.PAYOFF_MAX_CALL),
+                  'strike': 0.9 + 0.01 * i,
+                  'df': np.concatenate([[1.0], np.exp(-0.03 * t)]),
+                  'log_shift': (0.03 - 0.5 * vol**2) * t,
+                  'log_scale': float(vol)})
+  ex = list(range(steps))
+  calib = n // 2 if n > 2 else None
+  v, res, ranks = lsm.price_shared(w.t(), ex, items, 2, 7, calib, dev,
+                                   basis_log=2)
+  for i in (0, 7, 15, 16):
+    v1, r1, k1 = lsm.price_shared(w.t(), ex, items[i:i + 1], 2, 7, calib,
+                                  dev, basis_log=2)
+    assert torch.equal(v1[0], v[i]) and torch.equal(r1[0], res[i])
+    assert torch.equal(k1[0], ranks[i])
+    it = dict(items[i], log_shift=None)
+    shift = torch.as_tensor(items[i]['log_shift'], device=dev).reshape(-1, 1)
+    log_s = shift + items[i]['log_scale'] * w
+    _, r2, _ = lsm.price_shared(log_s.t(), ex, [it], 2, 7, calib, dev,
+                                basis_log=2)
+    if n > 4:  # a handful of rows fits every path: no stable regression
+      np.testing.assert_allclose(_np(r2[0]), _np(res[i]), rtol=1e-12)
+
+
+def test_shared_paths_exponential_and_monomial_mask():
+  # one date: the values are the payoffs, so exp(shift + scale x) is seen
+  # directly; range reduction and the degree-13 sum leave 2 ulp (4.5e-16)
+  x = torch.linspace(-700.0, 700.0, 100001, dtype=torch.float64,
+                     device='cuda')
+  it = {'payoff': lsm.PAYOFF_MAX_CALL, 'strike': 0.0, 'df': np.ones(2)}
+  v, _, _ = lsm.price_shared(x.reshape(-1, 1), [0], [it], 2, 7, None,
+                             x.device, basis_log=2)
+  want = np.exp(_np(x))
+  assert np.max(np.abs(_np(v[0]) / want - 1)) <= 4.5e-16
+  # the constant alone (mask 1): the continuation is the mean of the
+  # in-the-money rows
+  s = torch.tensor([[90.0, 80.0], [95.0, 120.0], [105.0, 70.0],
+                    [85.0, 99.0]], dtype=torch.float64, device='cuda')
+  it = {'payoff': lsm.PAYOFF_BASKET_PUT, 'strike': 100.0, 'df': np.ones(3)}
+  v, _, ranks = lsm.price_shared(s, [0, 1], [it], 2, 1, None, s.device)
+  last = np.maximum(100 - _np(s)[:, 1], 0)
+  first = np.maximum(100 - _np(s)[:, 0], 0)
+  cont = last[first > 0].mean()
+  np.testing.assert_allclose(_np(v[0]), np.where(first > cont, first, last),
+                             rtol=1e-15)
+  assert int(ranks[0, 0]) == 1

@@ -83,6 +83,12 @@ class Lsm(ctypes.Structure):
               ('stride_asset', _i64)]
 
 
+class LsmItem(ctypes.Structure):
+  _fields_ = [('payoff', _i32), ('pad0', _i32), ('strike', _f64),
+              ('payoff_table', _c_void_p), ('df', _c_void_p),
+              ('log_shift', _c_void_p), ('log_scale', _f64)]
+
+
 class Contract(ctypes.Structure):
   _fields_ = [('kind', _i32), ('n_steps', _i32), ('stream_id', _u32),
               ('greeks_mode', _i32), ('n_paths', _i64),
@@ -160,6 +166,11 @@ _SIGS = {
     'tqf_batch_price': (_i32, [_c_void_p, _i32, _c_void_p, _c_void_p, _i32,
                                _c_void_p, _c_void_p, _u64, _i32, _i32, _i32,
                                _c_void_p, _c_void_p, _c_void_p]),
+    'tqf_lsm_shared_workspace_size': (_i64, [_i64, _i32, _i32]),
+    'tqf_lsm_price_shared': (_i32, [ctypes.POINTER(Lsm), _c_void_p, _i32,
+                                    _i32, _c_void_p, _i32, _c_void_p,
+                                    _c_void_p, _c_void_p, _c_void_p,
+                                    _c_void_p]),
     'tqf_lsm_price': (_i32, [ctypes.POINTER(Lsm), _c_void_p, _i32, _c_void_p,
                              _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                              _c_void_p, _c_void_p]),

@@ -10,15 +10,13 @@ with r = -ln(df)/T; each option is then priced by least_square_mc with the
 degree-2 polynomial basis on ln S and the call/put payoff on S
 (utils.py:137-167), and the result is scaled back by the spot.
 
-Here the unit paths come from the exact GBM kernel (tqf_gbm_exact) with
-the engine's antithetic Philox stream (the reference's
-STATELESS_ANTITHETIC), the per-option mapping to ln(S / S0) is one
-elementwise pass on the GPU, and the regression runs in the FP64 LSM
-kernels (tqf_lsm_price on log prices: basis on ln S, payoff on S).  The
-options' regressions are independent: each runs on its own stream (up to
-four, default priority), so one option's single-workgroup solves overlap
-the other options' bandwidth-bound date passes, and the prices come back
-in one copy.  A user basis_fn falls back to the torch LSM with the same
+Here the Brownian paths W(t) come from the fused kernel's constant-
+coefficient model with the engine's antithetic Philox stream (the
+reference's STATELESS_ANTITHETIC), and the options are regressed together
+in the FP64 one-asset LSM kernels (tqf_lsm_price_shared: basis on ln S,
+payoff on S), one launch per exercise date.  ln(S / S0) is an affine map of
+W(t) per option and date, which the standardised basis does not see, so the
+kernels read W itself and no option has paths of its own.  A user basis_fn falls back to the torch LSM with the same
 log-path / payoff split.
 """
 import numpy as np
@@ -31,19 +29,6 @@ from tqf.models import longstaff_schwartz as lsm_lib
 from tqf.models import utils
 
 __all__ = ['bs_lsm_price']
-
-
-_STREAMS = {}
-_MAX_STREAMS = 4
-
-
-def _streams(dev, n):
-  """Up to _MAX_STREAMS side streams of `dev` (default priority), cached."""
-  key = str(dev)
-  pool = _STREAMS.setdefault(key, [])
-  while len(pool) < min(n, _MAX_STREAMS):
-    pool.append(torch.cuda.Stream(device=dev))
-  return pool[:min(n, _MAX_STREAMS)]
 
 
 def _vec(v, n, dtype):
@@ -63,6 +48,8 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
   dev = _native.device()
   spots_np = np.asarray(utils.to_numpy(spots), np.float64).reshape(-1)
   n_opt = spots_np.shape[0]
+  if n_opt == 0:
+    raise ValueError('`spots` holds no option')
   expiry = _vec(expiry_times, n_opt, dtype)
   strike = _vec(strikes, n_opt, dtype) / spots_np
   vol = _vec(volatility, n_opt, dtype)
@@ -84,38 +71,42 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
                    np.zeros(1), int(num_samples), rng, torch.float64,
                    mode='store', dev=dev)[:, 0, :]
   w = w_t.t()  # [N, T]
-  t = torch.as_tensor(times, dtype=torch.float64, device=dev).reshape(1, -1)
-  t_t = t.t()
   ex = list(range(int(num_exercise_times)))
   if basis_fn is None:
     basis_fn = lsm_lib.make_polynomial_basis(2)
   bspec = getattr(basis_fn, '_tqf_basis', None)
   if bspec is not None and bspec[0] == 'poly':
-    main = torch.cuda.current_stream(dev)
-    streams = _streams(dev, n_opt)
-    outs = []
-    for b in range(n_opt):
-      st = streams[b % len(streams)]
-      st.wait_stream(main)  # the unit paths are written on the caller's
-      with torch.cuda.stream(st):
-        dfs = np.exp(-rate[b] * times * expiry[b])
-        kind = (lsm_lib.PAYOFF_MAX_CALL if call[b]
-                else lsm_lib.PAYOFF_BASKET_PUT)
-        # ln(S / S0) in one pass: the LSM kernels take log prices
-        # (basis on ln S, payoff on exp)
-        log_s_t = torch.add((rate[b] - 0.5 * vol[b]**2) * (t_t * expiry[b]),
-                            w_t, alpha=float(vol[b] * np.sqrt(expiry[b])))
+    degree = bspec[1]
+    kind = lambda b: (lsm_lib.PAYOFF_MAX_CALL if call[b]
+                      else lsm_lib.PAYOFF_BASKET_PUT)
+    dfs = lambda b: np.exp(-rate[b] * times * expiry[b])
+    shift = lambda b: (rate[b] - 0.5 * vol[b]**2) * (times * expiry[b])
+    scale = lambda b: float(vol[b] * np.sqrt(expiry[b]))
+    if lsm_lib.shared_supported(1, degree, int(num_samples),
+                                num_calibration_samples):
+      items = [{'payoff': kind(b), 'strike': strike[b],
+                'df': np.concatenate([[1.0], dfs(b)]), 'log_shift': shift(b),
+                'log_scale': scale(b)} for b in range(n_opt)]
+      _, res, _ = lsm_lib.price_shared(
+          w, ex, items, degree, (2 << degree) - 1, num_calibration_samples,
+          dev, basis_log=2)
+      prices = res[:, 0].cpu().numpy()
+    else:
+      outs = []
+      for b in range(n_opt):
+        log_s_t = torch.add(
+            torch.as_tensor(shift(b), device=dev).reshape(-1, 1), w_t,
+            alpha=scale(b))
         # [N, T, 1] view of [T][1][N] memory
-        paths = log_s_t.unsqueeze(1).permute(2, 0, 1)
         outs.append(lsm_lib._native_lsm(
-            paths, ex, (kind, np.array([strike[b]])), bspec[1],
-            np.concatenate([[1.0], dfs]).reshape(-1, 1, 1),
+            log_s_t.unsqueeze(1).permute(2, 0, 1), ex,
+            (kind(b), np.array([strike[b]])), degree,
+            np.concatenate([[1.0], dfs(b)]).reshape(-1, 1, 1),
             num_calibration_samples, torch.float64, dev, basis_log=2))
-    for st in streams:
-      main.wait_stream(st)
-    prices = torch.cat(outs).cpu().numpy()
+      prices = torch.cat(outs).cpu().numpy()
     return torch.as_tensor(prices * spots_np, dtype=dtype, device=dev)
   prices = []
+  t = torch.as_tensor(times, dtype=torch.float64, device=dev).reshape(1, -1)
   for b in range(n_opt):
     dfs = np.exp(-rate[b] * times * expiry[b])
     log_s = ((vol[b] * np.sqrt(expiry[b])) * w +

@@ -174,6 +174,71 @@ def step_major_f64(paths):
   return out.permute(2, 0, 1)
 
 
+_SHARED_MAX_ITEMS, _SHARED_MAX_DEGREE = 16, 4
+
+
+def shared_supported(dim, degree, n_paths, num_calib):
+  """Whether price_shared takes these sizes (others run payoff by payoff)."""
+  return (dim == 1 and degree <= _SHARED_MAX_DEGREE and
+          n_paths > int(num_calib or 0))
+
+
+def price_shared(paths, ex, items, degree, mask, num_calib, dev,
+                 basis_log=0, path_discounts=None):
+  """Prices several payoffs on the same one-asset paths, one launch per
+  exercise date for all of them (tqf_lsm_price_shared).
+
+  paths: float64 [N, T] with any strides.  items: dicts with payoff, strike,
+  df [n_ex + 1] (padded), and optionally table [T, N] (contiguous) or
+  log_shift [n_ex] and log_scale (basis_log 2: the log price at date e is
+  log_shift[e] + log_scale * stored value).  mask: bit m set when the
+  monomial of exponent m is in the basis.  Returns (values [B, N] at the
+  first exercise date, results [B, 2], ranks [B, max(n_ex - 1, 1)])."""
+  n, nt = paths.shape
+  l = _native.Lsm()
+  l.paths = paths.data_ptr()
+  l.stride_path, l.stride_time = paths.stride()
+  l.stride_asset = 1
+  l.n_paths, l.n_times, l.dim = n, nt, 1
+  l.degree, l.basis_log = degree, int(basis_log)
+  l.num_calibration = int(num_calib or 0)
+  l.rcond = 10 * bin(mask).count('1') * np.finfo(np.float64).eps
+  if path_discounts is not None:
+    l.path_discounts = path_discounts.data_ptr()
+  n_ex, nb = len(ex), len(items)
+  exi = (ctypes.c_int32 * n_ex)(*ex)
+  values = torch.empty((nb, n), dtype=torch.float64, device=dev)
+  results = torch.empty((nb, 2), dtype=torch.float64, device=dev)
+  ranks = torch.empty((nb, max(n_ex - 1, 1)), dtype=torch.int32, device=dev)
+  if n_ex < 2:
+    ranks.zero_()
+  for b0 in range(0, nb, _SHARED_MAX_ITEMS):
+    part = items[b0:b0 + _SHARED_MAX_ITEMS]
+    arr = (_native.LsmItem * len(part))()
+    keep = []
+    for o, it in zip(arr, part):
+      o.payoff, o.strike = it['payoff'], float(it['strike'])
+      host = [np.ascontiguousarray(it['df'], np.float64)]
+      o.df = host[0].ctypes.data
+      if it.get('table') is not None:
+        o.payoff_table = it['table'].data_ptr()
+      if it.get('log_shift') is not None:
+        host.append(np.ascontiguousarray(it['log_shift'], np.float64))
+        o.log_shift = host[1].ctypes.data
+        o.log_scale = float(it['log_scale'])
+      keep.append(host)
+    ws = torch.empty(int(_native.lib().tqf_lsm_shared_workspace_size(
+        n, len(part), n_ex)) // 8 + 1, dtype=torch.float64, device=dev)
+    _native.call('tqf_lsm_price_shared', ctypes.byref(l), arr,
+                 ctypes.c_int32(len(part)), ctypes.c_int32(mask), exi,
+                 ctypes.c_int32(n_ex), ctypes.c_void_p(ws.data_ptr()),
+                 ctypes.c_void_p(values[b0].data_ptr()),
+                 ctypes.c_void_p(results[b0].data_ptr()),
+                 ctypes.c_void_p(ranks[b0].data_ptr()),
+                 _native.stream_ptr(dev))
+  return values, results, ranks
+
+
 def _native_lsm(x, ex, pspec, degree, df, num_calib, dtype, dev,
                 return_details=False, basis_log=False, exponents=None,
                 path_values=None):
@@ -212,6 +277,34 @@ def _native_lsm(x, ex, pspec, degree, df, num_calib, dtype, dev,
                               'basis functions')
   expo_t = torch.as_tensor(expo, device=dev).contiguous()
   n = paths_b.shape[1]
+  if shared_supported(d, degree, n, num_calib) and bp == 1 and (
+      k <= degree + 1) and not (per_path and df.shape[2] > 1):
+    # one asset, shared paths: every payoff in the same launches
+    p64 = step_major_f64(paths_b[0])
+    pdb = None
+    dfs = None
+    if per_path:
+      col = df[:, :, 0]  # [n_ex + 1, N]
+      pdb = torch.as_tensor(col, dtype=torch.float64, device=dev).contiguous()
+    else:
+      dfn = df.cpu().numpy() if torch.is_tensor(df) else df
+      dfs = np.broadcast_to(dfn, dfn.shape[:-1] + (n_batch,)).reshape(
+          dfn.shape[0], -1, n_batch)[:, 0]
+    items = []
+    for b in range(n_batch):
+      it = {'payoff': kind,
+            'strike': strikes[b if strikes.shape[0] > 1 else 0],
+            'df': np.ones(df.shape[0]) if per_path else dfs[:, b]}
+      if table is not None:
+        it['table'] = table[:, b if table.shape[1] > 1 else 0, :].T.contiguous()
+      items.append(it)
+    mask = int(np.bitwise_or.reduce(1 << expo[:, 0].astype(np.int64)))
+    values, res, ranks = price_shared(p64[:, :, 0], ex, items, degree, mask,
+                                      num_calib, dev, basis_log, pdb)
+    if path_values is not None:
+      path_values.copy_(values[-1])
+    out = res[:, 0].to(dtype)
+    return (out, res[:, 1].clone(), ranks) if return_details else out
   ws = torch.empty(int(_native.lib().tqf_lsm_workspace_size(n, k)) // 8 + 1,
                    dtype=torch.float64, device=dev)
   cash = torch.empty(n, dtype=torch.float64, device=dev)
