@@ -444,6 +444,30 @@ int tqf_lsm_final(const double* cash, const double* vals, double df0,
                   int64_t first, int64_t n, double* workspace, double* result,
                   void* stream);
 
+/* ---- Bermudan swaption inputs (one-factor Hull-White) -------------------- */
+
+/* Device arrays; slot[i] is the exercise index (each once, 0 .. n_ex - 1) of
+ * simulation date i or -1; entries first[u n_payoffs + b] .. first[u
+ * n_payoffs + b + 1] - 1 hold (C, G, w) of payoff b at exercise date u: its
+ * value is max(1 - sum w exp(C - r G), 0), or 0 without entries. */
+typedef struct tqf_swaption_plan {
+  int32_t n_dates, n_ex, n_payoffs, pad0;
+  const double* dt;       /* [n_dates] step length before each date          */
+  const int32_t* slot;    /* [n_dates]                                       */
+  const int32_t* first;   /* [n_ex * n_payoffs + 1]                          */
+  const double* entries;  /* [.][3]                                          */
+} tqf_swaption_plan;
+
+/* Short rates (path p, date i at rates[p stride_path + i stride_time]) to
+ * the regression's inputs, float64 and date-major: short_rate [n_ex][n],
+ * payoff [n_payoffs][n_ex][n], discounts [n_ex + 1][n] (row 0 = 1, row u + 1
+ * = exp(-sum of r dt up to exercise date u)).  Every exercise index must
+ * have its date: rows without one are not written. */
+int tqf_swaption_inputs(const void* rates, int64_t stride_path,
+                        int64_t stride_time, int64_t n_paths, int32_t dtype,
+                        const tqf_swaption_plan* plan, double* short_rate,
+                        double* payoff, double* discounts, void* stream);
+
 /* ---- MLP continuation value (6 -> 64 -> 64 -> 1, SiLU) ------------------ */
 
 /* Parameters: float32 [4673] = W1[6][64] | b1[64] | W2[64][64] | b2[64] |

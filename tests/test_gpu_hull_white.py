@@ -219,3 +219,41 @@ def test_time_dependent_mean_reversion_takes_the_euler_route():
   d = _np(model._drift_fn(torch.tensor(0.7, dtype=torch.float64), x))
   want = 0.0 + a * 0.01 + s * s / 2 / a * (1 - np.exp(-2 * a * 0.7)) - a * 0.02
   np.testing.assert_allclose(d, want, rtol=1e-12)
+
+
+@pytest.mark.parametrize('n,dtype', [(2, torch.float64), (257, torch.float64),
+                                     (1025, torch.float64),
+                                     (1025, torch.float32)])
+def test_swaption_inputs_kernel_matches_the_tensor_operations(n, dtype):
+  # swaptions whose later dates are padded at the maturity (merged and zero
+  # weights, a date with no payment left), rates date-major and path-major,
+  # path counts around a workgroup: the kernel's price against the tensor
+  # route on the same rates.  float64: sums of up to 8 bonds in another
+  # order, 1e-15 each, through a 3 x 3 solve, 1e-11; float32 rates: the
+  # tensor route rounds bonds and payoffs to float32 (6e-8 each, swap values
+  # of about 1e-2 from terms near 1: 1e-5 relative), 1e-3
+  print('swaption inputs', n, dtype, flush=True)
+  base = 1.0 + 0.5 * np.arange(9)
+  at = lambda i: base[min(i, 8)]
+  ex = np.array([[at(k + i) for i in range(8)] for k in (0, 2, 5)])
+  start = np.array([[[at(k + i + j) for j in range(8)] for i in range(8)]
+                    for k in (0, 2, 5)])
+  end = np.clip(start + 0.5, 0.0, 5.0)
+  model = tqf.models.hull_white.HullWhiteModel1F(0.03, 0.01, _flat,
+                                                 dtype=dtype)
+  plan = sw._plan(ex, end, 0.1)
+  rates = model.sample_paths(plan['sim_times'], num_samples=n,
+                             random_type=RandomType.STATELESS, seed=[n, 1])
+  dcf, cpn = end - start, 0.011 * np.ones_like(end)
+  want = _np(sw._price_on_paths(plan, sw._exercise_bonds(model, plan, rates,
+                                                         end),
+                                rates, end, dcf, cpn,
+                                tqf.models.longstaff_schwartz.
+                                make_polynomial_basis(2), dtype))
+  view = rates.permute(1, 2, 0).contiguous().permute(2, 0, 1)
+  tol = 1e-11 if dtype == torch.float64 else 1e-3
+  for r in (rates, view):
+    got = _np(sw._price_native(model, plan, r, end, dcf, cpn, 2, dtype))
+    if n > 4:  # a handful of rows fits every path: no stable regression
+      np.testing.assert_allclose(got, want, rtol=tol)
+    assert np.all(np.isfinite(got))

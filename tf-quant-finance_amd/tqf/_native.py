@@ -89,6 +89,12 @@ class LsmItem(ctypes.Structure):
               ('log_shift', _c_void_p), ('log_scale', _f64)]
 
 
+class SwaptionPlan(ctypes.Structure):
+  _fields_ = [('n_dates', _i32), ('n_ex', _i32), ('n_payoffs', _i32),
+              ('pad0', _i32), ('dt', _c_void_p), ('slot', _c_void_p),
+              ('first', _c_void_p), ('entries', _c_void_p)]
+
+
 class Contract(ctypes.Structure):
   _fields_ = [('kind', _i32), ('n_steps', _i32), ('stream_id', _u32),
               ('greeks_mode', _i32), ('n_paths', _i64),
@@ -166,6 +172,9 @@ _SIGS = {
     'tqf_batch_price': (_i32, [_c_void_p, _i32, _c_void_p, _c_void_p, _i32,
                                _c_void_p, _c_void_p, _u64, _i32, _i32, _i32,
                                _c_void_p, _c_void_p, _c_void_p]),
+    'tqf_swaption_inputs': (_i32, [_c_void_p, _i64, _i64, _i64, _i32,
+                                   ctypes.POINTER(SwaptionPlan), _c_void_p,
+                                   _c_void_p, _c_void_p, _c_void_p]),
     'tqf_lsm_shared_workspace_size': (_i64, [_i64, _i32, _i32]),
     'tqf_lsm_price_shared': (_i32, [ctypes.POINTER(Lsm), _c_void_p, _i32,
                                     _i32, _c_void_p, _i32, _c_void_p,

@@ -213,6 +213,14 @@ class HullWhiteModel1F:
                    normal_draws=None, validate_args=False, name=None):
     """Short-rate paths [num_samples, len(times), 1]."""
     del name
+    return self._sample(times, num_samples, random_type, seed, skip,
+                        time_step, times_grid, normal_draws, validate_args,
+                        'paths')
+
+  def _sample(self, times, num_samples, random_type, seed, skip, time_step,
+              times_grid, normal_draws, validate_args, mode):
+    """sample_paths; mode 'view' gives the same values as a view of the
+    coalesced date-major store (the exact route)."""
     times_np = np.asarray(utils.to_numpy(times), np.float64)
     if times_np.ndim != 1:
       raise ValueError('`times` should be a rank 1 Tensor. '
@@ -253,7 +261,7 @@ class HullWhiteModel1F:
     spec = ('hull_white', self._kernel_constants)
     return engine.run(spec, all_times, mask, times_np.shape[0],
                       torch.zeros(1, dtype=self._dtype, device=dev),
-                      int(num_samples), rng, self._dtype, mode='paths',
+                      int(num_samples), rng, self._dtype, mode=mode,
                       dev=dev)
 
   def _bond_constants(self, times, maturities):

@@ -3,17 +3,22 @@ Longstaff-Schwartz on simulated short rates (mirror of
 tff.models.hull_white.bermudan_swaption_price,
 tff/models/hull_white/swaption.py:314-724; payoff mapping :876-935).
 
-The short rate runs in the fused kernel (HullWhiteModel1F); at every
-exercise date the swap's value per path comes from zero-coupon bonds
+The short rate runs in the fused kernel (HullWhiteModel1F) and, with a
+polynomial basis, the regression's inputs in one more (tqf_swaption_inputs);
+a user basis takes the tensor operations below.  At every exercise date the swap's value per path comes from zero-coupon bonds
 reconstituted from r(t) (fixed leg sum_j c_j tau_j P(t, T_j), floating leg
 1 - P(t, T_n)); the path discount factor is prod exp(-r_k dt_k) on the
 simulation grid (the rate at the end of each interval, as the reference
 does); the regression is on a polynomial basis of r(t) at the union of all
 swaptions' exercise dates, every swaption of the batch one payoff column.
 """
+import ctypes
+
 import numpy as np
 import torch
 
+from tqf import _native
+from tqf.engine import euler as engine
 from tqf.models import longstaff_schwartz as lsm
 from tqf.models import utils
 from tqf.models.hull_white.one_factor import HullWhiteModel1F
@@ -78,11 +83,16 @@ def bermudan_swaption_price(*, exercise_times, floating_leg_start_times,
   model = HullWhiteModel1F(mean_reversion, volatility,
                            initial_discount_rate_fn=reference_rate_fn,
                            dtype=tdt)
-  r_t = model.sample_paths(plan['sim_times'], num_samples=num_samples,
-                           random_type=random_type, seed=seed, skip=skip)
-  bonds = _exercise_bonds(model, plan, r_t, pay)
   basis = lsm.make_polynomial_basis(2) if lsm_basis is None else lsm_basis
-  value = _price_on_paths(plan, bonds, r_t, pay, dcf, cpn, basis, tdt)
+  bspec = getattr(basis, '_tqf_basis', None)
+  r_t = model._sample(plan['sim_times'], num_samples, random_type, seed, skip,
+                      None, None, None, False, 'view')
+  if (bspec is not None and bspec[0] == 'poly' and
+      lsm.shared_supported(1, bspec[1], int(r_t.shape[0]), None)):
+    value = _price_native(model, plan, r_t, pay, dcf, cpn, bspec[1], tdt)
+  else:
+    bonds = _exercise_bonds(model, plan, r_t, pay)
+    value = _price_on_paths(plan, bonds, r_t, pay, dcf, cpn, basis, tdt)
   value = torch.as_tensor(notional, dtype=tdt, device=r_t.device) * value
   if plan['batch_shape']:
     return value.reshape(plan['batch_shape'])
@@ -104,6 +114,78 @@ def _plan(ex, pay, time_step):
               ex_index=ex_index.reshape(ex.shape), ex_full=ex_full,
               sim_times=sim_times, tau=tau, curve_times=curve_times,
               n_ex=ex.shape[-1])
+
+
+def _payoff_entries(model, plan, pay, dcf, cpn):
+  """(first [n_u * B + 1], entries [., 3]) of tqf_swaption_inputs: per
+  exercise date of the union and swaption, the constants (C, G) of its
+  payment dates' bonds P = exp(C - r G) and their weights."""
+  shape = np.broadcast_shapes(pay.shape, plan['ex_full'].shape)
+  n_ex, n_pay = shape[-2:]
+  flat_b = int(np.prod(plan['batch_shape'])) if plan['batch_shape'] else 1
+  f0, p0big, g, y = model._bond_constants(plan['ex_full'], pay)
+  c = np.log(p0big) + f0 * g - 0.5 * y * g * g
+  w = np.broadcast_to(cpn * dcf, shape).reshape(flat_b, n_ex, n_pay).copy()
+  w[..., -1] += 1.0
+  c, g = (np.broadcast_to(a, shape).reshape(flat_b, n_ex, n_pay)
+          for a in (c, g))
+  exi = plan['ex_index'].reshape(flat_b, n_ex)
+  n_u = plan['unique_ex'].shape[0]
+  first, entries = [0], []
+  for u in range(n_u):
+    for b in range(flat_b):
+      own = np.flatnonzero(exi[b] == u)
+      if own.size:
+        e = own[-1]
+        merged = {}
+        for j in range(n_pay):
+          key = (c[b, e, j], g[b, e, j])
+          merged[key] = merged.get(key, 0.0) + w[b, e, j]
+        own_entries = [k + (v,) for k, v in merged.items() if v != 0.0]
+        # a swap with no payment left still has its own date
+        entries += own_entries or [(0.0, 0.0, 0.0)]
+      first.append(len(entries))
+  return (np.asarray(first, np.int32),
+          np.asarray(entries, np.float64).reshape(-1, 3))
+
+
+def _price_native(model, plan, r_t, pay, dcf, cpn, degree, tdt):
+  """Prices [batch] from the short rates [N, k, 1]: the regression's inputs
+  in one kernel (tqf_swaption_inputs), then the one-asset LSM chain with
+  every swaption in the same launches."""
+  dev = r_t.device
+  sim_times, unique_ex = plan['sim_times'], plan['unique_ex']
+  n, n_u = r_t.shape[0], unique_ex.shape[0]
+  flat_b = int(np.prod(plan['batch_shape'])) if plan['batch_shape'] else 1
+  slot = np.full(sim_times.shape[0], -1, np.int32)
+  slot[np.searchsorted(sim_times, unique_ex)] = np.arange(n_u)
+  first, entries = _payoff_entries(model, plan, pay, dcf, cpn)
+  pl = _native.SwaptionPlan()
+  pl.n_dates, pl.n_ex, pl.n_payoffs = sim_times.shape[0], n_u, flat_b
+  keep = []
+  stage = engine.Staging(dev)
+  stage.add(np.concatenate([[0.0], np.diff(sim_times)]), torch.float64,
+            [(pl, 'dt')])
+  stage.add(slot, torch.int32, [(pl, 'slot')])
+  stage.add(first, torch.int32, [(pl, 'first')])
+  stage.add(entries, torch.float64, [(pl, 'entries')])
+  stage.flush(keep)
+  f64 = dict(dtype=torch.float64, device=dev)
+  rate = torch.empty((n_u, n), **f64)
+  table = torch.empty((flat_b, n_u, n), **f64)
+  disc = torch.empty((n_u + 1, n), **f64)
+  _native.call('tqf_swaption_inputs', ctypes.c_void_p(r_t.data_ptr()),
+               ctypes.c_int64(r_t.stride(0)), ctypes.c_int64(r_t.stride(1)),
+               ctypes.c_int64(n), ctypes.c_int32(_native.dtype_code(tdt)),
+               ctypes.byref(pl), ctypes.c_void_p(rate.data_ptr()),
+               ctypes.c_void_p(table.data_ptr()),
+               ctypes.c_void_p(disc.data_ptr()), _native.stream_ptr(dev))
+  items = [{'payoff': lsm.PAYOFF_TABLE, 'strike': 1.0, 'table': table[b],
+            'df': np.ones(n_u + 1)} for b in range(flat_b)]
+  _, res, _ = lsm.price_shared(rate.t(), list(range(n_u)), items, degree,
+                               (2 << degree) - 1, None, dev,
+                               path_discounts=disc)
+  return res[:, 0].to(tdt)
 
 
 def _exercise_bonds(model, plan, r_t, pay):
