@@ -146,11 +146,14 @@ __device__ __forceinline__ int row_slot(double v) {
 template <typename R, int MODEL>
 struct Stepper {
   static constexpr int D = ModelDim<MODEL>::D;
+  // pv: the Heston vol-of-vol factors a.p[3], a.p[4], which the caller may
+  // hold in vector registers
   __device__ __forceinline__ static void step(const EulerArgs<R>& a, R* x,
                                               const R* z, R dt, R sdt,
                                               const R* tab, int lv_row,
                                               R lv_w, int i,
-                                              const StepRow<R>& row) {
+                                              const StepRow<R>& row,
+                                              const R* pv) {
     if (MODEL == TQF_MODEL_GBM) {
       const R drift = a.p[0] * x[0];
       const R vol = a.p[1] * x[0];
@@ -172,7 +175,7 @@ struct Stepper {
       const R ssq = sq * sdt;
       x[0] = fma_r(vp, row.c[0], x[0]);
       x[1] = fma_r(vp, row.c[2], x[1] + row.c[1]);
-      const R c1 = fma_r(a.p[4], z[1], a.p[3] * z[0]);
+      const R c1 = fma_r(pv[1], z[1], pv[0] * z[0]);
       x[0] = fma_r(ssq, z[0], x[0]);
       x[1] = fma_r(ssq, c1, x[1]);
     } else if (MODEL == TQF_MODEL_HULL_WHITE) {
@@ -280,7 +283,11 @@ __device__ __forceinline__ void record(const EulerArgs<R>& a, R* lds_pay,
 }
 
 template <typename R, int MODEL, int RNG, bool kStage>
-__global__ void __launch_bounds__(kBlock) euler_kernel(EulerArgs<R> a) {
+// float32: eight waves per SIMD.  Without the bound the Sobol kernels take
+// 106 scalar registers, which allow seven, and a launch of 2,048 workgroups
+// (eight per CU) runs its last 256 in a round of their own.
+__global__ void __launch_bounds__(kBlock, sizeof(R) == 4 ? 8 : 1)
+euler_kernel(EulerArgs<R> a) {
   constexpr int D = ModelDim<MODEL>::D;
   extern __shared__ __align__(16) unsigned char lds[];
   R* lds_pay = (R*)(lds + a.lds_pay_off);
@@ -365,6 +372,11 @@ __global__ void __launch_bounds__(kBlock) euler_kernel(EulerArgs<R> a) {
 
   int lv_row = 0;
   const int n_dims = a.n_steps * D;
+  // vector registers: a scalar operand halves an instruction's issue rate
+  R pv[2] = {a.p[3], a.p[4]};
+  if constexpr (sizeof(R) == 4 && (MODEL == TQF_MODEL_HESTON_FT ||
+                                   MODEL == kModelHestonOwn))
+    asm volatile("" : "+v"(pv[0]), "+v"(pv[1]));
   auto fetch = [&](int i, R* z) {
     if (D == 2) {
       nrm.get2(a.rng, i, z);
@@ -411,7 +423,8 @@ __global__ void __launch_bounds__(kBlock) euler_kernel(EulerArgs<R> a) {
           lv_w = t <= t0 ? (R)0 : fast_div(t - t0, t1 - t0);
         }
       }
-      Stepper<R, MODEL>::step(a, x, zc, dt, sdt, tab, lv_row, lv_w, i, row);
+      Stepper<R, MODEL>::step(a, x, zc, dt, sdt, tab, lv_row, lv_w, i, row,
+                              pv);
       if (s >= 0) {
         const R off = kHasStepRow<MODEL> ? row.c[3] : (R)0;
         if constexpr (kStage)
@@ -780,7 +793,8 @@ euler_tangent_kernel(EulerArgs<R> a, TangentArgs<R> t) {
         T[1][D + 3] += sq * (t.rho * dw0 + s1r * dw1);         // xi
         T[1][D + 4] += t.xi * sq * (dw0 - t.rho / s1r * dw1);  // rho
       }
-      Stepper<R, MODEL>::step(a, x, z, dt, sdt, nullptr, 0, (R)0, i, row);
+      Stepper<R, MODEL>::step(a, x, z, dt, sdt, nullptr, 0, (R)0, i, row,
+                              a.p + 3);
       if (s >= 0) rec(s, ld_uniform(a.t_next, i));
     }
   }

@@ -63,24 +63,29 @@ constexpr int sobol_lds_words(int D) { return 2 * kSobolChunk * D; }
 // ---- float32 shifted-Sobol inverse CDF (piecewise cubic, table in LDS) ----
 // z = Phi^-1((n + 1/2) 2^-25) of the top 25 bits n of a 32-bit point.  The
 // point folds onto the lower half with its sign mask s (m = (v ^ s) >> 7 in
-// [0, 2^24); the upper half, s all ones, reads the negated copy of the
-// table); the float32 value of m * 128 (exact, formed by masking the low 7
+// [0, 2^24)); the float32 value of m * 128 (exact, formed by masking the low 7
 // bits) indexes a segment by its exponent and top 3 mantissa bits, and its
 // low 20 mantissa bits minus 2^20 are the cubic's variable (csrc/
 // fit_icdf.py derives the table; exhaustive float32 error: 5.2e-7
 // absolute, 3.3e-7 relative for |z| >= 1e-3).
 //
+// The cubic runs on the mantissa bits placed as the float h in [1, 1.125):
+// h - 1.125 is 2^-23 times that variable, exactly, and the staged
+// coefficients carry the powers of 2^23, so every step's result is the same
+// bits as with the integer variable at one conversion less.  The upper half's
+// sign is put on the result.
+//
 // LDS image: segment k sits at byte ((k + 1072) & 255) * 16, which is bits
 // 20..27 of the float's bit pattern times 16 (one AND of its upper half):
 // segments 0..191 land on bytes [768, 3840), and m = 0 (the float 0) on
-// byte 0, which holds the constant kIcdfZero.  The negated copy is 4096
-// bytes above (bit 12, set from the sign mask with one AND-OR).
-constexpr int kIcdfHalf = 4096;
+// byte 0, which holds the constant kIcdfZero.  One copy for both halves: a
+// wave's reads of the few segments near the centre, which hold most points,
+// then meet on the same entries (no bank conflict) whatever their signs.
+constexpr int kIcdfLdsBytes = 4096;
 constexpr int kIcdfSlot0 = (134 << kIcdfSegBits) & 255;  // 48
-constexpr int kIcdfLdsBytes = 2 * kIcdfHalf;
 static_assert(kIcdfSegBits == 3, "the LDS addressing assumes 8 sub-segments");
-static_assert((kIcdfSlot0 + kIcdfSegs) * 16 <= kIcdfHalf,
-              "a table half must fit below bit 12");
+static_assert((kIcdfSlot0 + kIcdfSegs) * 16 <= kIcdfLdsBytes,
+              "the table must fit below bit 12");
 
 // The table's block-shared copy (static LDS of every kernel that uses it).
 __device__ __forceinline__ unsigned char* icdf_lds() {
@@ -88,37 +93,55 @@ __device__ __forceinline__ unsigned char* icdf_lds() {
   return t;
 }
 
-// Cooperative copy of both halves into LDS (caller synchronises).
+// Cooperative copy into LDS (caller synchronises).
 __device__ __forceinline__ void icdf_stage(unsigned char* lds) {
   float4* t = (float4*)lds;
-  for (int e = threadIdx.x; e < kIcdfSegs; e += blockDim.x) {
-    const float4 c = make_float4(kIcdfCoef[4 * e], kIcdfCoef[4 * e + 1],
-                                 kIcdfCoef[4 * e + 2], kIcdfCoef[4 * e + 3]);
-    t[kIcdfSlot0 + e] = c;
-    t[kIcdfHalf / 16 + kIcdfSlot0 + e] = make_float4(-c.x, -c.y, -c.z, -c.w);
-  }
-  if (threadIdx.x == 0) {
-    t[0] = make_float4(kIcdfZero, 0.f, 0.f, 0.f);
-    t[kIcdfHalf / 16] = make_float4(-kIcdfZero, 0.f, 0.f, 0.f);
-  }
+  for (int e = threadIdx.x; e < kIcdfSegs; e += blockDim.x)
+    t[kIcdfSlot0 + e] =
+        make_float4(kIcdfCoef[4 * e], kIcdfCoef[4 * e + 1] * 0x1p23f,
+                    kIcdfCoef[4 * e + 2] * 0x1p46f,
+                    kIcdfCoef[4 * e + 3] * 0x1p69f);
+  if (threadIdx.x == 0) t[0] = make_float4(kIcdfZero, 0.f, 0.f, 0.f);
 }
 
+// The transform's masks in vector registers: as scalar operands or literals
+// of three-input instructions they would halve the issue rate (see
+// PhiloxKeys).
+struct IcdfMasks {
+  uint32_t top25, low20, one, sign;
+
+  __device__ __forceinline__ void init() {
+    top25 = 0xFFFFFF80u;
+    low20 = 0x000FFFFFu;
+    one = 0x3F800000u;
+    sign = 0x80000000u;
+    asm volatile("" : "+v"(top25), "+v"(low20), "+v"(one), "+v"(sign));
+  }
+};
+
 __device__ __forceinline__ float icdf_shifted_f32(uint32_t v,
-                                                  const unsigned char* lds) {
+                                                  const unsigned char* lds,
+                                                  const IcdfMasks& k) {
   const uint32_t s = (uint32_t)((int32_t)v >> 31);
-  const uint32_t w = (v ^ s) & 0xFFFFFF80u;       // m * 128
+  // m * 128 = (v ^ s) & top25
+  const uint32_t w = __builtin_amdgcn_bitop3_b32(v, s, k.top25, 0x28);
   const uint32_t fi = __float_as_uint((float)w);  // exact
   // m * 128 is 0 or in [2^7, 2^31): exponent 134..157, so bits 20..27 of
-  // fi are 48..239 (no wrap), or 0 for m = 0; the offset stays in its half
+  // fi are 48..239 (no wrap), or 0 for m = 0
   uint32_t off;  // (fi >> 16) & 0xFF0: one AND reading the upper half-word
   asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD "
       "src0_sel:WORD_1 src1_sel:DWORD"
       : "=v"(off)
       : "v"(fi), "v"(0xFF0u));
-  const float g = (float)(int32_t)(fi | 0xFFF00000u);  // [-2^20, -1]
-  const float4 c = *(const float4*)(lds + ((s & (uint32_t)kIcdfHalf) | off));
-  return __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c.w, g, c.z), g, c.y),
-                        g, c.x);
+  // (fi & low20) | one, as a float less 1.125: [-2^-3, -2^-23]
+  const float g = __uint_as_float(__builtin_amdgcn_bitop3_b32(
+                      fi, k.low20, k.one, 0xEA)) - 1.125f;
+  const float4 c = *(const float4*)(lds + off);
+  const float z = __builtin_fmaf(
+      __builtin_fmaf(__builtin_fmaf(c.w, g, c.z), g, c.y), g, c.x);
+  // z with the sign of s: z ^ (s & sign)
+  return __uint_as_float(__builtin_amdgcn_bitop3_b32(
+      __float_as_uint(z), s, k.sign, 0x78));
 }
 
 // Bytes of dynamic LDS the normal source of a kernel needs (the Sobol
@@ -146,6 +169,7 @@ struct Normals {
   int chunk_base;
   int D;  // normals per step
   unsigned char* icdf;
+  IcdfMasks masks;
   uint32_t* hx;
   __amdgpu_buffer_rsrc_t lo_rsrc;  // low-byte table (raw buffer, bounds-checked)
   u32x2 lo_next;                   // get2: the next step's low-byte words
@@ -164,6 +188,7 @@ struct Normals {
     if constexpr (kIcdf) {
       icdf = icdf_lds();
       icdf_stage(icdf);
+      masks.init();
     }
     if (RNG == TQF_RNG_PHILOX_ANTITHETIC) {
       const int64_t half = a.n_paths / 2;
@@ -248,7 +273,7 @@ struct Normals {
     if constexpr (RNG == TQF_RNG_SOBOL) {
       return sobol_ref_normal<R>(v, a.sscale);
     } else if constexpr (kIcdf) {
-      return (R)icdf_shifted_f32(v, icdf);
+      return (R)icdf_shifted_f32(v, icdf, masks);
     } else {
       return sobol_shifted_normal(v, R(0));
     }

@@ -396,8 +396,10 @@ sobol_normals_run_kernel(const uint32_t* __restrict__ v, int dim, R scale,
                          R* __restrict__ out, int dw, int rpw) {
   constexpr bool kF32 = sizeof(R) == sizeof(float);
   unsigned char* icdf = nullptr;
+  IcdfMasks masks;
   if constexpr (kF32) {
     icdf = icdf_lds();
+    masks.init();
     if (mode == 1) {
       icdf_stage(icdf);
       __syncthreads();
@@ -409,7 +411,7 @@ sobol_normals_run_kernel(const uint32_t* __restrict__ v, int dim, R scale,
               if (mode == 0)
                 z = sobol_ref_normal<R>(x, scale);
               else if constexpr (kF32)
-                z = (R)icdf_shifted_f32(x, icdf);
+                z = (R)icdf_shifted_f32(x, icdf, masks);
               else
                 z = sobol_shifted_normal(x, R(0));
               out[i * dim + d] = z;
