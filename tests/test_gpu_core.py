@@ -589,6 +589,46 @@ def test_shifted_normal_transform_exhaustive():
     assert err[~big].max() <= 2e-10
 
 
+@pytest.mark.parametrize('nd', [1, 2, 5, 8, 13, 23, 24, 25])
+def test_reference_normal_transform_exhaustive(nd):
+  # dimension 0 with nd digits is the bit reversal of the index: indices
+  # 0 .. 2^nd - 1 put every nd-digit point through the kernel (25: the last
+  # size beyond the 24-digit table)
+  import ctypes
+  from tqf import _native
+  n = 2**nd
+  v = tsobol.device_columns(1, nd)
+  out = torch.empty(n, dtype=torch.float32, device='cuda')
+  _native.call('tqf_sobol_normals', _native.ptr(v), ctypes.c_int32(1),
+               ctypes.c_int32(nd), ctypes.c_int64(n), ctypes.c_int64(0),
+               None, ctypes.c_int32(0), ctypes.c_int32(_native.TQF_F32),
+               _native.ptr(out), _native.stream_ptr(out.device))
+  got = _np(out).astype(np.float64)
+  k = np.arange(n, dtype=np.uint64)
+  rev = np.zeros(n, np.uint64)
+  for b in range(nd):
+    rev |= ((k >> np.uint64(b)) & np.uint64(1)) << np.uint64(nd - 1 - b)
+  u = rev.astype(np.float64) * 2.0**-nd
+  mid, inner = u == 0.5, (u > 0) & (u != 0.5)
+  assert (got[mid] == 0).all() and mid.sum() == 1
+  if nd <= 24:
+    assert (got[u == 0] == -np.inf).all()
+    # relative: the cubics with their float32 coefficients 5.62e-8, the last
+    # rounding 2^-24 = 5.96e-8, the roundings before it scaled by |h| <= 2^-4
+    want = onormal.quasi_normals(u[inner])
+    assert (np.abs(got[inner] - want) <= 1.25e-7 * np.abs(want)).all()
+  else:
+    # u is rounded to 24 bits above 1/2, which moves z by up to
+    # 2^-25 / phi(z) = 8.9e-6 at u = 0.999
+    inner &= u < 0.999
+    want = onormal.quasi_normals(u[inner])
+    assert (np.abs(got[inner] - want) <= 1e-5).all()
+  # odd about u = 1/2, bit for bit
+  order = np.argsort(rev)[1:]
+  if nd <= 24:
+    np.testing.assert_array_equal(got[order], -got[order][::-1])
+
+
 def test_euler_shifted_sobol_parity():
   # fused float32 Heston FT with the shifted-Sobol stream against the
   # oracle driven by the same points through the exact inverse CDF

@@ -596,11 +596,12 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
     a.lds_spot_off = (int)((sums + 15) & ~(size_t)15);
     pay = (size_t)a.lds_spot_off + (size_t)kWaves * kWave * sizeof(R);
   }
-  size_t lds = (size_t)rng_lds_bytes(r->kind, D);
+  const int rng_kind = kernel_rng<R>(r);
+  size_t lds = (size_t)rng_lds_bytes(rng_kind, D);
   if (m->kind == TQF_MODEL_LOCAL_VOL) {
     const int64_t lv = (int64_t)m->lv_nt * m->lv_nx * (int64_t)sizeof(R);
     const int64_t total = (int64_t)((lds + lv + 15) & ~(size_t)15) +
-                          (int64_t)pay + kIcdfLdsBytes;
+                          (int64_t)pay + kDyadicLdsBytes;
     a.lv_in_lds = lv <= kMaxLvLdsBytes && total <= 64 * 1024;
     if (a.lv_in_lds) lds += (size_t)lv;
   }
@@ -615,7 +616,7 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
                        ? kModelHestonOwn
                        : m->kind;
 #define TQF_PICK(MODEL, RNG) \
-  if (kind == MODEL && r->kind == RNG)                                   \
+  if (kind == MODEL && rng_kind == RNG)                                  \
     kern = stage ? euler_kernel<R, MODEL, RNG, true>                     \
                  : euler_kernel<R, MODEL, RNG, false>;
 #define TQF_PICK_RNG(MODEL)                       \
@@ -623,7 +624,10 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   TQF_PICK(MODEL, TQF_RNG_PHILOX)                 \
   TQF_PICK(MODEL, TQF_RNG_PHILOX_ANTITHETIC)      \
   TQF_PICK(MODEL, TQF_RNG_SOBOL)                  \
-  TQF_PICK(MODEL, TQF_RNG_SOBOL_SHIFTED)
+  TQF_PICK(MODEL, TQF_RNG_SOBOL_SHIFTED)          \
+  if constexpr (sizeof(R) == sizeof(float)) {     \
+    TQF_PICK(MODEL, kRngSobolDyadic)              \
+  }
   TQF_PICK_RNG(TQF_MODEL_GBM)
   TQF_PICK_RNG(TQF_MODEL_CONST)
   TQF_PICK_RNG(TQF_MODEL_HESTON_FT)

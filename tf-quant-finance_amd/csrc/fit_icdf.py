@@ -23,8 +23,16 @@ Each cubic is a weighted least-squares fit (weight 1/max(|z|, 1e-3)),
 sharpened towards minimax by Lawson's iteration, over every m of the
 segment; segments of octaves with at most 4 points interpolate them.  The
 whole table is then checked exhaustively over all 2^24 values of m with
-the float32 Horner evaluation.  Run: python fit_icdf.py  (writes
-icdf_table.h next to this file and prints the error bounds).
+the float32 Horner evaluation.
+
+A second table (icdf_dyadic_table.h) serves the reference transform of
+unshifted points, erfinv((u - 1/2) 2) sqrt 2 at u = v 2^-nd, nd <= 24: with y
+= t 2^-24 the point folded onto (0, 1/2], z = Phi^-1(y) as a function of the
+float32 value of t 2^8, 16 sub-segments to an octave, the constant of the
+segment that ends at y = 1/2 held at zero.
+
+Run: python fit_icdf.py  (writes icdf_table.h and icdf_dyadic_table.h next
+to this file and prints the error bounds).
 """
 import os
 
@@ -87,6 +95,68 @@ def horner_f32(c32, seg, g):
   return p
 
 
+DYADIC_BITS = 4
+N_DYADIC = 23 << DYADIC_BITS
+
+
+def fit_to_zero(g, z, iters=30):
+  """fit_segment with c0 = 0 (the segment that ends at y = 1/2)."""
+  sc = -float(g.min())
+  x = g / sc
+  v = np.stack([x, x * x, x**3], 1)
+  base = 1.0 / np.maximum(np.abs(z), 1e-6)
+  wt = np.ones_like(x) / x.size
+  for _ in range(iters):
+    w = np.sqrt(wt) * base
+    cc, *_ = np.linalg.lstsq(v * w[:, None], z * w, rcond=None)
+    e = np.abs(v @ cc - z) * base
+    wt = wt * (e + 1e-6 * e.max())
+    wt /= wt.sum()
+  return np.concatenate([[0.0], cc / sc**np.arange(1, 4)])
+
+
+def dyadic_main():
+  low = 23 - DYADIC_BITS
+  t = np.arange(1, 2**23, dtype=np.int64)
+  fi = (t * 256).astype(np.float32).view(np.uint32).astype(np.int64)
+  seg = (fi >> low) - ((127 + 8) << DYADIC_BITS)
+  g = ((fi & ((1 << low) - 1)) - (1 << low)).astype(np.float64)
+  z = special.ndtri(t * 2.0**-24)
+  bounds = np.searchsorted(seg, np.arange(N_DYADIC + 1))
+  coef = np.zeros((N_DYADIC, 4))
+  for s in range(N_DYADIC):
+    sl = slice(bounds[s], bounds[s + 1])
+    if bounds[s + 1] > bounds[s]:
+      fit = fit_to_zero if s == N_DYADIC - 1 else fit_segment
+      coef[s] = fit(g[sl], z[sl])
+  # the kernel's variable is 2^-23 g: exact powers of two
+  c32 = coef.astype(np.float32)
+  err = np.abs(horner_f32(c32, seg, g) - z)
+  bound = ('max abs err %.2e, max rel err %.2e, rms rel err %.2e' % (
+      err.max(), (err / np.abs(z)).max(), np.sqrt(np.mean((err / z)**2))))
+  print('dyadic: ' + bound)
+  out = os.path.join(os.path.dirname(os.path.abspath(__file__)),
+                     'icdf_dyadic_table.h')
+  with open(out, 'w') as f:
+    f.write('// Generated by fit_icdf.py: piecewise-cubic Phi^-1(t 2^-24) on '
+            't in [1, 2^23),\n// segment s = (bits(float(t * 256)) >> 19) - '
+            '2160, variable h in [-2^-4, -2^-23],\n'
+            '// z = ((c3 h + c2) h + c1) h + c0.  Exhaustive float32 check:\n'
+            '// %s.\n' % bound)
+    f.write('#pragma once\n\nnamespace tqf {\n\n')
+    f.write('constexpr int kDyadicSegBits = %d;\n'
+            'constexpr int kDyadicSegs = %d;\n\n' % (DYADIC_BITS, N_DYADIC))
+    f.write('// {c0, c1, c2, c3} per segment\n')
+    f.write('__device__ __constant__ const float '
+            'kDyadicCoef[kDyadicSegs * 4] = {\n')
+    for s in range(N_DYADIC):
+      f.write('    ' + ', '.join(
+          '%sf' % float(v * 2.0**(23 * k)).hex()
+          for k, v in enumerate(c32[s].astype(np.float64))) + ',\n')
+    f.write('};\n\n}  // namespace tqf\n')
+  print('wrote', out)
+
+
 def main():
   m, seg, g, z = segments()
   order = np.argsort(seg, kind='stable')
@@ -131,3 +201,4 @@ def main():
 
 if __name__ == '__main__':
   main()
+  dyadic_main()

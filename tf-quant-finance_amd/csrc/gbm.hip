@@ -150,6 +150,11 @@ int launch_d(const GbmArgs<R>& a, int rng_kind, unsigned blocks, size_t lds,
       hipLaunchKernelGGL((gbm_exact_kernel<R, TQF_RNG_PHILOX_ANTITHETIC, MAXD>),
                          blocks, kPathBlock, lds, s, a);
       break;
+    case kRngSobolDyadic:
+      if constexpr (sizeof(R) == sizeof(float))
+        hipLaunchKernelGGL((gbm_exact_kernel<R, kRngSobolDyadic, MAXD>),
+                           blocks, kPathBlock, lds, s, a);
+      break;
     case TQF_RNG_SOBOL:
       hipLaunchKernelGGL((gbm_exact_kernel<R, TQF_RNG_SOBOL, MAXD>), blocks,
                          kPathBlock, lds, s, a);
@@ -181,17 +186,18 @@ int launch(const tqf_gbm* g, const tqf_grid* grid, const tqf_rng* r,
   a.mode = mode;
   a.out = (R*)out;
   a.n_paths = n_paths;
-  size_t lds = ((size_t)rng_lds_bytes(r->kind, g->dim) + 15) & ~(size_t)15;
+  const int rng_kind = kernel_rng<R>(r);
+  size_t lds = ((size_t)rng_lds_bytes(rng_kind, g->dim) + 15) & ~(size_t)15;
   a.stage_off = (int)lds;
   a.stage_recs = kStageWords / g->dim;  // dim <= 16: at least 2
   if (mode == TQF_OUT_PATH_MAJOR)
     lds += (size_t)kPathBlock * kStageStride * sizeof(R);
   if (lds == 0) lds = 16;
   const unsigned blocks = (unsigned)((n_paths + kPathBlock - 1) / kPathBlock);
-  if (g->dim <= 1) return launch_d<R, 1>(a, r->kind, blocks, lds, s);
-  if (g->dim <= 4) return launch_d<R, 4>(a, r->kind, blocks, lds, s);
-  if (g->dim <= 8) return launch_d<R, 8>(a, r->kind, blocks, lds, s);
-  return launch_d<R, 16>(a, r->kind, blocks, lds, s);
+  if (g->dim <= 1) return launch_d<R, 1>(a, rng_kind, blocks, lds, s);
+  if (g->dim <= 4) return launch_d<R, 4>(a, rng_kind, blocks, lds, s);
+  if (g->dim <= 8) return launch_d<R, 8>(a, rng_kind, blocks, lds, s);
+  return launch_d<R, 16>(a, rng_kind, blocks, lds, s);
 }
 
 }  // namespace

@@ -14,6 +14,7 @@
 #pragma once
 
 #include "common.h"
+#include "icdf_dyadic_table.h"
 #include "icdf_table.h"
 
 namespace tqf {
@@ -35,6 +36,7 @@ struct RngArgs {
   const uint32_t* sshift;  // [ndims] or null
   int64_t sfirst;          // sequence index of path 0
   R sscale;                // 2^-nd
+  int sshl;                // 32 - nd
   int64_t n_paths;         // antithetic split
 };
 
@@ -53,6 +55,7 @@ inline void fill_rng_args(RngArgs<R>& a, const tqf_rng* r, int64_t n_paths) {
   a.sshift = r->sobol_shift;
   a.sfirst = r->sobol_first_index;
   a.sscale = (R)std::ldexp(1.0, -r->sobol_nd);
+  a.sshl = 32 - r->sobol_nd;
   a.n_paths = n_paths;
 }
 
@@ -144,10 +147,85 @@ __device__ __forceinline__ float icdf_shifted_f32(uint32_t v,
       __float_as_uint(z), s, k.sign, 0x78));
 }
 
+// ---- float32 reference transform of points of at most 24 digits -----------
+// z = Phi^-1(v 2^-nd), the value of erfinv((u - 1/2) 2) sqrt 2, by the same
+// scheme: V = v << (32 - nd), folded onto the lower half as W = V or 2^32 - V
+// (at most 24 significant bits, an exact float), 16 sub-segments to an octave
+// (csrc/fit_icdf.py).  Without a branch and about half the instructions of
+// erfinv_f32, whose tail polynomial runs in a third of the waves; exhaustive
+// error 1.2e-7 relative (erfinv_f32: 3.0e-7), root mean square 3.5e-8
+// (8.5e-8).  Recording 365 states of 2^19 Heston paths (1.53 GB): 392 us,
+// with erfinv_f32 443.  More than 24 digits (sequences beyond 2^24 points)
+// have no exact float W and keep erfinv_f32.
+//
+// LDS image: the segment of bits 19..27 of the float at that number times
+// 16; V = 2^31 (u = 1/2) reads zeros, V = 0 the constant -inf.
+constexpr int kRngSobolDyadic = 16;  // kernel-internal code of this transform
+constexpr int kDyadicLdsBytes = 8192;
+constexpr int kDyadicSlot0 = (135 << kDyadicSegBits) & 511;  // 112
+static_assert(kDyadicSegBits == 4 && kDyadicSlot0 + kDyadicSegs < 512,
+              "the LDS addressing assumes 16 sub-segments");
+
+__device__ __forceinline__ unsigned char* dyadic_lds() {
+  __shared__ __align__(16) unsigned char t[kDyadicLdsBytes];
+  return t;
+}
+
+// Cooperative copy into LDS (caller synchronises).
+__device__ __forceinline__ void dyadic_stage(unsigned char* lds) {
+  float4* t = (float4*)lds;
+  for (int e = threadIdx.x; e < kDyadicSegs; e += blockDim.x)
+    t[kDyadicSlot0 + e] =
+        make_float4(kDyadicCoef[4 * e], kDyadicCoef[4 * e + 1],
+                    kDyadicCoef[4 * e + 2], kDyadicCoef[4 * e + 3]);
+  if (threadIdx.x == 0) {
+    t[0] = make_float4(-INFINITY, 0.f, 0.f, 0.f);
+    t[kDyadicSlot0 + kDyadicSegs] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+}
+
+struct DyadicMasks {
+  uint32_t low19, one, sign;
+
+  __device__ __forceinline__ void init() {
+    low19 = 0x0007FFFFu;
+    one = 0x3F800000u;
+    sign = 0x80000000u;
+    asm volatile("" : "+v"(low19), "+v"(one), "+v"(sign));
+  }
+};
+
+__device__ __forceinline__ float dyadic_f32(uint32_t v, int shl,
+                                            const unsigned char* lds,
+                                            const DyadicMasks& k) {
+  const uint32_t V = v << shl;
+  const uint32_t s = (uint32_t)((int32_t)V >> 31);
+  const uint32_t fi = __float_as_uint((float)((V ^ s) - s));  // exact
+  // (fi & low19) | one, as a float less 1.0625: [-2^-4, -2^-23]
+  const float g = __uint_as_float(__builtin_amdgcn_bitop3_b32(
+                      fi, k.low19, k.one, 0xEA)) - 1.0625f;
+  const float4 c = *(const float4*)(lds + ((fi >> 15) & 0x1FF0u));
+  const float z = __builtin_fmaf(
+      __builtin_fmaf(__builtin_fmaf(c.w, g, c.z), g, c.y), g, c.x);
+  return __uint_as_float(__builtin_amdgcn_bitop3_b32(
+      __float_as_uint(z), s, k.sign, 0x78));
+}
+
+// The kernel's code for rng kind `kind`: the table transform where it
+// applies.
+template <typename R>
+inline int kernel_rng(const tqf_rng* r) {
+  return sizeof(R) == sizeof(float) && r->kind == TQF_RNG_SOBOL &&
+                 r->sobol_nd <= 24
+             ? kRngSobolDyadic
+             : r->kind;
+}
+
 // Bytes of dynamic LDS the normal source of a kernel needs (the Sobol
-// high-bit words; the ICDF table is static LDS).
+// high-bit words; the inverse-CDF tables are static LDS).
 __host__ __device__ constexpr int rng_lds_bytes(int rng_kind, int D) {
-  return (rng_kind == TQF_RNG_SOBOL || rng_kind == TQF_RNG_SOBOL_SHIFTED)
+  return (rng_kind == TQF_RNG_SOBOL || rng_kind == TQF_RNG_SOBOL_SHIFTED ||
+          rng_kind == kRngSobolDyadic)
              ? sobol_lds_words(D) * 4
              : 0;
 }
@@ -155,7 +233,9 @@ __host__ __device__ constexpr int rng_lds_bytes(int rng_kind, int D) {
 template <typename R, int RNG>
 struct Normals {
   static constexpr bool kSobol =
-      RNG == TQF_RNG_SOBOL || RNG == TQF_RNG_SOBOL_SHIFTED;
+      RNG == TQF_RNG_SOBOL || RNG == TQF_RNG_SOBOL_SHIFTED ||
+      RNG == kRngSobolDyadic;
+  static constexpr bool kDyadic = RNG == kRngSobolDyadic;
   static constexpr bool kIcdf =
       RNG == TQF_RNG_SOBOL_SHIFTED && sizeof(R) == sizeof(float);
   static constexpr bool kPhilox =
@@ -170,6 +250,7 @@ struct Normals {
   int D;  // normals per step
   unsigned char* icdf;
   IcdfMasks masks;
+  DyadicMasks dmasks;
   uint32_t* hx;
   __amdgpu_buffer_rsrc_t lo_rsrc;  // low-byte table (raw buffer, bounds-checked)
   u32x2 lo_next;                   // get2: the next step's low-byte words
@@ -189,6 +270,11 @@ struct Normals {
       icdf = icdf_lds();
       icdf_stage(icdf);
       masks.init();
+    }
+    if constexpr (kDyadic) {
+      icdf = dyadic_lds();
+      dyadic_stage(icdf);
+      dmasks.init();
     }
     if (RNG == TQF_RNG_PHILOX_ANTITHETIC) {
       const int64_t half = a.n_paths / 2;
@@ -274,6 +360,8 @@ struct Normals {
       return sobol_ref_normal<R>(v, a.sscale);
     } else if constexpr (kIcdf) {
       return (R)icdf_shifted_f32(v, icdf, masks);
+    } else if constexpr (kDyadic) {
+      return (R)dyadic_f32(v, a.sshl, icdf, dmasks);
     } else {
       return sobol_shifted_normal(v, R(0));
     }

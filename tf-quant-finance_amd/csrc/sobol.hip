@@ -391,27 +391,34 @@ sobol_points_run_kernel(const uint32_t* __restrict__ v, int dim, double scale,
 template <typename R>
 __global__ void __launch_bounds__(256)
 sobol_normals_run_kernel(const uint32_t* __restrict__ v, int dim, R scale,
-                         int64_t n, int64_t first,
+                         int shl, int64_t n, int64_t first,
                          const uint32_t* __restrict__ shift, int mode,
                          R* __restrict__ out, int dw, int rpw) {
   constexpr bool kF32 = sizeof(R) == sizeof(float);
   unsigned char* icdf = nullptr;
   IcdfMasks masks;
+  DyadicMasks dmasks;
+  // float32: mode 1 the shifted transform's table, mode 0 the reference
+  // transform's where the points have at most 24 digits (shl >= 8)
   if constexpr (kF32) {
-    icdf = icdf_lds();
     masks.init();
-    if (mode == 1) {
+    dmasks.init();
+    icdf = mode == 1 ? icdf_lds() : dyadic_lds();
+    if (mode == 1)
       icdf_stage(icdf);
-      __syncthreads();
-    }
+    else if (shl >= 8)
+      dyadic_stage(icdf);
+    __syncthreads();
   }
   sobol_run(v, dim, n, first, shift, dw, rpw,
             [&](int64_t i, int d, uint32_t x) {
               R z;
-              if (mode == 0)
+              if constexpr (kF32) {
+                z = mode == 1  ? (R)icdf_shifted_f32(x, icdf, masks)
+                    : shl >= 8 ? (R)dyadic_f32(x, shl, icdf, dmasks)
+                               : sobol_ref_normal<R>(x, scale);
+              } else if (mode == 0)
                 z = sobol_ref_normal<R>(x, scale);
-              else if constexpr (kF32)
-                z = (R)icdf_shifted_f32(x, icdf, masks);
               else
                 z = sobol_shifted_normal(x, R(0));
               out[i * dim + d] = z;
@@ -523,12 +530,14 @@ extern "C" int tqf_sobol_normals(const uint32_t* v, int32_t dim, int32_t nd,
   const RunGrid g = run_grid(dim, n, first_index);
   if (dtype == TQF_F32) {
     hipLaunchKernelGGL(sobol_normals_run_kernel<float>, g.grid, dim3(256), 0,
-                       (hipStream_t)stream, v, dim, std::ldexp(1.0f, -nd), n,
-                       first_index, shift, mode, (float*)out, g.dw, g.rpw);
+                       (hipStream_t)stream, v, dim, std::ldexp(1.0f, -nd),
+                       32 - nd, n, first_index, shift, mode, (float*)out, g.dw,
+                       g.rpw);
   } else {
     hipLaunchKernelGGL(sobol_normals_run_kernel<double>, g.grid, dim3(256), 0,
-                       (hipStream_t)stream, v, dim, std::ldexp(1.0, -nd), n,
-                       first_index, shift, mode, (double*)out, g.dw, g.rpw);
+                       (hipStream_t)stream, v, dim, std::ldexp(1.0, -nd),
+                       32 - nd, n, first_index, shift, mode, (double*)out, g.dw,
+                       g.rpw);
   }
   return check_launch("tqf_sobol_normals");
 }
