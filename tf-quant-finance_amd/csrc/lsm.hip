@@ -47,14 +47,6 @@ __device__ __forceinline__ f64x4 mfma_f64(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Lane `l`'s value of v in every lane (l wave-uniform).
-__device__ __forceinline__ double read_lane_f64(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)b, l);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 struct LsmArgs {
   const double* paths;      // float64, element (p, t, j) at
                             // paths[p sp + t st + j sa]
@@ -1033,9 +1025,10 @@ bool moment_plan(int d, int deg, int n_pairs, MomentPlan* out) {
 // w of eight keeps tile rows 15 - w and w (17 tiles, two waves per SIMD so
 // they fit its registers).  Per panel p:
 //   1. the owner of tile (p, p) factors it in registers (16 sequential
-//      columns on one wave, operands exchanged between lanes, no LDS round
-//      and no workgroup barrier) and forms Y = L_pp^-1 in the same column
-//      steps, with zero rows and columns for dropped pivots;
+//      columns on one wave, operands exchanged between lanes by DPP row
+//      broadcasts and row swaps, no LDS round and no workgroup barrier) and
+//      forms Y = L_pp^-1 in the same column steps, with zero rows and
+//      columns for dropped pivots;
 //   2. each panel tile (a, p) becomes X = A_ap Y^T (4 MFMAs), staged in LDS;
 //   3. each trailing tile (a, b), a >= b > p, takes -= X_ap X_bp^T (4 MFMAs).
 // Two workgroup barriers per panel in place of one per column.  The back
@@ -1043,11 +1036,53 @@ bool moment_plan(int d, int deg, int n_pairs, MomentPlan* out) {
 // tile (b, c), c < b, subtracts L_bc^T w_b from r_c (one tile per c and
 // step, so the order of the sums is fixed; the tiles' row sums meet in LDS
 // and are added all at once).  beta = D w.
+//
+// Bound by its serial chain, not by the matrix rate: of 138 us at K = 243 the
+// column steps took 41, the trailing updates 33, the back solve 25 (each left
+// out in turn).  Row broadcasts in place of LDS-crossbar shuffles, rows above
+// the pivot skipped at compile time, the factored tile kept out of the
+// register tiles and all tile loads issued together: 131 us.
 constexpr int kSolveWaves = 8;
 constexpr int kSolveThreads = 64 * kSolveWaves;
 constexpr int kBT = 16;         // tile edge
 constexpr int kBLd = 17;        // LDS row stride of a staged tile (doubles)
 constexpr int kBTiles = 17;     // two tile rows per wave: 136 / 8
+
+// f(integral_constant<k>) for every k in order (DPP controls are immediates).
+template <typename F, int... k>
+__device__ __forceinline__ void for_each_index(
+    F&& f, std::integer_sequence<int, k...>) {
+  (f(std::integral_constant<int, k>{}), ...);
+}
+
+// v of lane k of the caller's row of 16 lanes.
+template <int k>
+__device__ __forceinline__ double row_lane_f64(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(
+      0, (int)(uint32_t)u, 0x150 + k, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(
+      0, (int)(uint32_t)(u >> 32), 0x150 + k, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// v of the same column of row g (of four) of 16 lanes: with both operands
+// equal, v_permlane16_swap leaves rows (0, 0, 2, 2) and (1, 1, 3, 3) and
+// v_permlane32_swap then repeats one half.
+template <int g>
+__device__ __forceinline__ uint32_t row_u32(uint32_t x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const uint32_t h = (g & 1) ? a[1] : a[0];
+  const auto b = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+  return (g & 2) ? b[1] : b[0];
+}
+template <int g>
+__device__ __forceinline__ double row_f64(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = row_u32<g>((uint32_t)u);
+  const uint32_t hi = row_u32<g>((uint32_t)(u >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
 
 __global__ void __launch_bounds__(kSolveThreads)
 lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
@@ -1108,19 +1143,27 @@ lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
     asm volatile("" : "+s"(wo));
   };
   f64x4 tile[kBTiles];
+  // every load issued before the first is used (the loads land in the
+  // tiles' own registers); entries past the matrix read G_00
 #pragma unroll
   for (int q = 0; q < kBTiles; ++q) {
     const int a = tile_a(q), b = tile_b(q);
-    f64x4 v = {0.0, 0.0, 0.0, 0.0};
-    if (a >= 0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
-        v[r] = (row < n && col < n)
-                   ? g[row * kext + col] * (dsc[row] * dsc[col]) : 0.0;
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
+      tile[q][r] = g[a >= 0 && row < n && col < n ? row * kext + col : 0];
     }
-    tile[q] = v;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int q = 0; q < kBTiles; ++q) {
+    const int a = tile_a(q), b = tile_b(q);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
+      tile[q][r] = a >= 0 && row < n && col < n
+                       ? tile[q][r] * (dsc[row] * dsc[col]) : 0.0;
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
@@ -1130,69 +1173,66 @@ lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
   // rows l / 16 + 4 r), together with Y_pp = L_pp^-1 (zero rows and columns
   // where a pivot is dropped).  The tile is symmetric and both triangles are
   // updated alike, so row k of the trailing square equals its column k.
-  // Column k: the pivot from its lane (v_readlane), its reciprocal root from
-  // v_rsq_f64 and two Newton steps, L_ik from lane 16 (l / 16) + k (the same
-  // row), L_jk = D_kj and the row k of R = I - (sum of the steps so far)
-  // from lane 16 (k % 4) + l % 16 (the same column); then
+  // Column k: the pivot and its reciprocal root, L_ik from lane
+  // 16 (l / 16) + k (the same row), L_jk = D_kj and the row k of R = I -
+  // (sum of the steps so far) from lane 16 (k % 4) + l % 16 (the same
+  // column); then
   // D_ij -= L_ik L_jk (i, j > k) and R_ij -= L_ik Y_kj (i > k) with
   // Y_kj = R_kj / L_kk, the forward substitution L Y = I done column by
   // column alongside the factorization.
-  auto factor_diag = [&](int pd) {
-    const int qd = pd < 8 ? 16 : pd;
-    f64x4 dv = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int q = 0; q < kBTiles; ++q)
-      if (q == qd) dv = tile[q];
+  // Only Y_pp and, of the last tile, the row of z are read later.
+  auto factor_diag = [&](int pd, f64x4 dv) {
     f64x4 yv;
 #pragma unroll
     for (int r = 0; r < 4; ++r) yv[r] = rl + 4 * r == cl ? 1.0 : 0.0;
     int kept = 0;
-#pragma unroll
-    for (int k = 0; k < kBT; ++k) {
-      const int rk = k >> 2, gk = k & 3, src = 16 * gk + cl;
-      const double dk = read_lane_f64(dv[rk], 16 * gk + k);
-      double dik[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) dik[r] = __shfl(dv[r], (lane & 48) + k, 64);
-      const double dkj = __shfl(dv[rk], src, 64);
-      const double rkj = __shfl(yv[rk], src, 64);
+    auto column = [&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      constexpr int rk = k >> 2, gk = k & 3;
+      // the lane's coordinates, opaque: the comparisons are made here rather
+      // than hoisted out of the panel loop, which would exhaust the registers
+      int rl_ = rl, cl_ = cl;
+      asm volatile("" : "+v"(rl_), "+v"(cl_));
+      const double dkj = row_f64<gk>(dv[rk]);
+      const double rkj = row_f64<gk>(yv[rk]);
+      const double dk = row_lane_f64<k>(dkj);
       const bool keep = kBT * pd + k < K && dk > thr && dk > 0;
-      double rinv = 0.0;
-      if (keep) {
-        double y = __builtin_amdgcn_rsq(dk);
-        y = y * fma(-0.5 * dk * y, y, 1.5);
-        y = y * fma(-0.5 * dk * y, y, 1.5);
-        rinv = y;
-      }
-      const double root = dk * rinv;  // 0 for a dropped pivot
+      // 1 / sqrt(dk): v_rsq_f64 (error e of about 2^-25), then one step of
+      // third order
+      const double y0 = __builtin_amdgcn_rsq(dk);
+      const double e = fma(-dk * y0, y0, 1.0);
+      const double y1 = fma(y0 * e, fma(0.375, e, 0.5), y0);
+      const double rinv = keep ? y1 : 0.0;
+      const double root = keep ? dk * y1 : 0.0;  // 0 for a dropped pivot
       kept += keep ? 1 : 0;
-      // branch-free: rinv = 0 leaves the updates no-ops and zeroes row and
-      // column k of L and Y
-      const double ljk = dkj * rinv, ykj = rkj * rinv;
+      // rinv = 0 leaves the updates no-ops and zeroes row and column k of L
+      // and Y.  Rows 4 r + rl with r < rk lie above row k for every lane and
+      // those with r > rk below it; only r == rk compares.
+      const double ljk = cl_ > k ? dkj * rinv : 0.0, ykj = rkj * rinv;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = rl + 4 * r;
-        const double lik = dik[r] * rinv;
-        double v = dv[r];
-        v = (i > k && cl > k) ? v - lik * ljk : v;
-        v = (cl == k && i > k) ? lik : v;
-        v = (cl == k && i == k) ? root : v;
+      for (int r = rk; r < 4; ++r) {
+        double lik = row_lane_f64<k>(dv[r]) * rinv;
+        if (r == rk) lik = rl_ > gk ? lik : 0.0;
+        double v = fma(-lik, ljk, dv[r]);
+        if (r == rk)
+          v = cl_ == k && rl_ >= gk ? (rl_ == gk ? root : lik) : v;
+        else
+          v = cl_ == k ? lik : v;
         dv[r] = v;
-        double y = yv[r];
-        y = i > k ? y - lik * ykj : y;
-        y = i == k ? ykj : y;
+        double y = fma(-lik, ykj, yv[r]);
+        if (r == rk) y = rl_ == gk ? ykj : y;
         yv[r] = y;
       }
-    }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for_each_index(column, std::make_integer_sequence<int, kBT>{});
 #pragma unroll
     for (int r = 0; r < 4; ++r) Ys[pd][(rl + 4 * r) * kBLd + cl] = yv[r];
-    // L_pp (lower, zero above) back into the register tile
+    if (pd == T - 1) {
 #pragma unroll
-    for (int q = 0; q < kBTiles; ++q)
-      if (q == qd)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          tile[q][r] = rl + 4 * r >= cl ? dv[r] : 0.0;
+      for (int r = 0; r < 4; ++r)
+        if (rl + 4 * r == K % kBT && cl < K % kBT) rv[kBT * pd + cl] = dv[r];
+    }
     if (lane == 0) rank_s += kept;
   };
   // p = -1 only factors tile (0, 0)
@@ -1244,11 +1284,17 @@ lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
     };
     if (next_owner) {
       const int qn = pn < 8 ? 16 : pn;
-      if (p >= 0)
+      f64x4 dv = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int q = 0; q < kBTiles; ++q)
-          if (q == qn) trail(q);
-      factor_diag(pn);
+      for (int q = 0; q < kBTiles; ++q)
+        if (q == qn) dv = tile[q];
+      if (p >= 0) {
+        const double* pa = P[pn];
+#pragma unroll
+        for (int s4 = 0; s4 < kBT; s4 += 4)
+          dv = mfma_f64(-pa[cl * kBLd + s4 + rl], pa[cl * kBLd + s4 + rl], dv);
+      }
+      factor_diag(pn, dv);
       refresh();
     }
     if (p >= 0)
@@ -1262,11 +1308,11 @@ lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
     // before its writes)
   }
   __syncthreads();
-  // r = z = row K of L
+  // r = z = row K of L (the last tile's part is there)
   const int bk = K / kBT, rk = K % kBT;
 #pragma unroll
   for (int q = 0; q < kBTiles; ++q)
-    if (tile_a(q) == bk)
+    if (tile_a(q) == bk && tile_b(q) < bk)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int col = kBT * tile_b(q) + cl;
