@@ -749,6 +749,41 @@ def test_heston_qe_parity(dtype, tol):
   _close(got[..., 1], want[..., 1], tol, scale=1e3 * np.max(want[..., 1]))
 
 
+@pytest.mark.parametrize('v0,theta', [(0.002, 0.05), (0.02, 0.002),
+                                      (0.2, 0.05)])
+def test_heston_qe_float32_variance_draw_far_out(v0, theta):
+  # one float32 step against the float64 step on the same draws, out to where
+  # 1 - Phi(z) has no float32 digits left (psi = 6.7, 11.2 and 1.04)
+  kappa, xi, dt = 1.2, 0.9, 0.25
+  zv = np.concatenate([np.linspace(-7, 8, 3001), [-0.9, -0.85, 6.5]])
+  z = np.stack([zv, np.zeros_like(zv)], -1)[:, None, :].astype(np.float32)
+  model = tqf.models.HestonModel(kappa, theta, xi, -0.6, dtype=torch.float32)
+  got = _np(model.sample_paths(np.array([dt]), [np.log(100.), v0],
+                               time_step=dt, normal_draws=z))[:, 0, 1]
+  want = oheston.update_variance(kappa, theta, xi, np.full(zv.shape, v0), dt,
+                                 z[:, 0, 0].astype(np.float64))
+  e = np.exp(-kappa * dt)
+  m = theta + (v0 - theta) * e
+  s2 = v0 * xi**2 * e / kappa * (1 - e) + theta * xi**2 / (
+      2 * kappa) * (1 - e)**2
+  psi = s2 / m**2
+  if psi < 1.5:
+    # vn = a (b + z)^2: a and b to a few ulp, the square's condition
+    b = np.sqrt(2 / psi - 1 + np.sqrt(2 / psi * (2 / psi - 1)))
+    a = m / (1 + b * b)
+    bound = a * 1e-6 * (b + np.abs(zv)) * (b + np.abs(b + zv)) + 1e-6 * want
+  else:
+    # vn = m (psi + 1) / 2 max(0, ln(2 / (psi + 1)) - ln Phi(-z)) (1 - Phi(z)
+    # has no float64 digits either at z = 8): a few float32 ulp of psi, and
+    # 2^-22 of the logarithm, 1e-2 of it above z = 6.5
+    from scipy import special
+    tail = special.log_ndtr(-z[:, 0, 0].astype(np.float64))
+    want = m * (psi + 1) / 2 * np.maximum(0, np.log(2 / (psi + 1)) - tail)
+    rel = 2.0**-22 + 1e-2 * (zv > 6.5)
+    bound = m * (psi + 1) / 2 * (1e-6 + rel * np.abs(tail)) + 1e-6 * want
+  assert (np.abs(got - want) <= bound).all()
+
+
 # --------------------------------------------------------------- Halton
 
 @pytest.mark.parametrize('dtype,rtol', [(torch.float32, 1e-6),

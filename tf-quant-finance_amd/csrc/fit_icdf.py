@@ -31,8 +31,12 @@ unshifted points, erfinv((u - 1/2) 2) sqrt 2 at u = v 2^-nd, nd <= 24: with y
 float32 value of t 2^8, 16 sub-segments to an octave, the constant of the
 segment that ends at y = 1/2 held at zero.
 
+The log of the normal tail (log2_normal_tail in common.h): a degree-13
+polynomial for log2(Phi(-z) e^(z^2 / 2)) on [-0.9, 6.5], minimax in the error
+of log2 Phi(-z) relative to max(1/2, its size).
+
 Run: python fit_icdf.py  (writes icdf_table.h and icdf_dyadic_table.h next
-to this file and prints the error bounds).
+to this file, prints the error bounds and the tail's coefficients).
 """
 import os
 
@@ -157,6 +161,29 @@ def dyadic_main():
   print('wrote', out)
 
 
+def tail_main(lo=-0.9, hi=6.5, deg=13, iters=80):
+  cheb, poly = np.polynomial.chebyshev, np.polynomial.polynomial
+  def want(z):
+    return np.log2(0.5 * special.erfcx(z / np.sqrt(2)))
+  z = lo + (hi - lo) * (1 - np.cos(np.pi * np.arange(4001) / 4000)) / 2
+  v = cheb.chebvander((2 * z - lo - hi) / (hi - lo), deg)
+  full = want(z) - z * z * 0.5 * np.log2(np.e)
+  w0 = 1 / np.maximum(0.5, np.abs(full))
+  wt = np.ones_like(z) / z.size
+  for _ in range(iters):
+    w = np.sqrt(wt) * w0
+    c, *_ = np.linalg.lstsq(v * w[:, None], want(z) * w, rcond=None)
+    e = np.abs(v @ c - want(z)) * w0
+    wt = wt * (e + 1e-3 * e.max())
+    wt /= wt.sum()
+  out = np.zeros(1)
+  for k in cheb.cheb2poly(c)[::-1]:
+    out = poly.polyadd(
+        poly.polymul(out, [-(lo + hi) / (hi - lo), 2 / (hi - lo)]), [k])
+  print('normal tail, fit %.1e:' % e.max(),
+        [float(x).hex() for x in out[:deg + 1].astype(np.float32)])
+
+
 def main():
   m, seg, g, z = segments()
   order = np.argsort(seg, kind='stable')
@@ -202,3 +229,4 @@ def main():
 if __name__ == '__main__':
   main()
   dyadic_main()
+  tail_main()
