@@ -471,3 +471,19 @@ def test_batch_short_contracts_and_item_counts_vs_oracle(greeks):
     for q, name in enumerate(batch_lib.GREEK_NAMES[c['kind']]):
       assert abs(r[name][0] - want[q]) <= 1e-5 * rms[q], (c['kind'], n, m,
                                                          name)
+
+
+@pytest.mark.parametrize('dtypes,shapes', [
+    (('float32',) * 3, ((), (1,), (1, 1))), (('float64',) * 3, ((),) * 3),
+    (('float32', 'float64', 'float32'), ((), (), (1,))),
+    (('float64',), ((),))])
+def test_parameter_values_read_together(dtypes, shapes):
+  # one gather and one read where types agree, each on its own otherwise:
+  # the values of float() either way
+  from tqf.engine import differentiable
+  vals = [0.1, -0.7, 1.0 / 3]
+  params = [torch.full(sh, v, dtype=getattr(torch, dt), device='cuda',
+                       requires_grad=True)
+            for v, dt, sh in zip(vals, dtypes, shapes)]
+  got = differentiable._values(params)
+  assert got == [float(p.detach().cpu().reshape(())) for p in params]

@@ -38,6 +38,18 @@ def _params(spec):
   return list(spec[1:1 + TANGENT_KINDS[spec[0]]])
 
 
+def _values(params):
+  """The scalar tensors' values.  A float() of a device tensor is a copy and
+  a wait each; tensors of one device and type are gathered on the device and
+  read in one."""
+  p0 = params[0]
+  if (len(params) > 1 and p0.is_cuda and p0.is_floating_point() and
+      all(p.device == p0.device and p.dtype == p0.dtype and p.numel() == 1
+          for p in params)):
+    return torch.stack([p.detach().reshape(()) for p in params]).tolist()
+  return [float(p) for p in params]
+
+
 def needs_gradients(spec, x0):
   """True when grad mode is on and the initial state or a parameter of the
   spec is a tensor that requires grad."""
@@ -57,7 +69,7 @@ class _Info:
     self.dtype, self.dev = dtype, dev
 
   def launch(self, x0, params):
-    vals = [float(p) for p in params]
+    vals = _values(params)
     spec = (self.spec[0],) + tuple(vals) + tuple(
         self.spec[1 + len(vals):])
     return engine.prepare(spec, self.all_times, self.keep_mask, self.k,
