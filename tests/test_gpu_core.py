@@ -749,6 +749,33 @@ def test_heston_qe_parity(dtype, tol):
   _close(got[..., 1], want[..., 1], tol, scale=1e3 * np.max(want[..., 1]))
 
 
+@pytest.mark.parametrize('n', [2**16 - 2, 2**16, 2**16 + 2])
+@pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
+@pytest.mark.parametrize('name', ['gbm', 'const', 'heston_ft', 'heston_own',
+                                  'local_vol'])
+def test_antithetic_rows_equal_path_major_records(name, dtype, n):
+  # 2^16 paths and more step both mirrors in one thread on coalesced rows;
+  # path-major records keep one path to a thread: the same bits
+  if name == 'local_vol':
+    times, x, vols = _lv_surface()
+    spec = ('local_vol', engine.LocalVolTable(times, x[0], x[1] - x[0], vols,
+                                              0.02))
+    x0 = [np.log(100.)]
+  elif name == 'heston_own':
+    spec, x0 = ('heston', 0.0, 2.0, 0.04, 0.3, -0.7, 1.0), [np.log(100.), 0.04]
+  else:
+    spec, _, x0 = _models()[name]
+  all_times = np.linspace(0.0, 1.0, 8)
+  keep = np.array([True, False, True, False, False, True, True, True])
+  rng = engine.RngSpec.from_random_type(mvn.RandomType.STATELESS_ANTITHETIC,
+                                        [4, 9], 0)
+  x0 = np.asarray(x0)[None, :] + 1e-3 * np.arange(n)[:, None] / n
+  run = lambda mode: engine.run(spec, all_times, keep, 5, x0, n, rng, dtype,
+                                mode=mode)
+  np.testing.assert_array_equal(_np(run('store').permute(2, 0, 1)),
+                                _np(run('paths')))
+
+
 @pytest.mark.parametrize('v0,theta', [(0.002, 0.05), (0.02, 0.002),
                                       (0.2, 0.05)])
 def test_heston_qe_float32_variance_draw_far_out(v0, theta):

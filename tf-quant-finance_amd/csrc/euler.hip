@@ -301,7 +301,11 @@ __device__ __forceinline__ void record(const EulerArgs<R>& a, R* lds_pay,
   }
 }
 
-template <typename R, int MODEL, int RNG, bool kStage>
+constexpr int64_t kPairMinPaths = 1 << 16;  // see launch
+
+// kPair (antithetic Philox normals, coalesced records): a thread steps path p
+// and its mirror p + n_paths / 2 with the normals drawn once.
+template <typename R, int MODEL, int RNG, bool kStage, bool kPair = false>
 // float32: eight waves per SIMD.  Without the bound the Sobol kernels take
 // 106 scalar registers, which allow seven, and a launch of 2,048 workgroups
 // (eight per CU) runs its last 256 in a round of their own.
@@ -311,9 +315,11 @@ euler_kernel(EulerArgs<R> a) {
   extern __shared__ __align__(16) unsigned char lds[];
   R* lds_pay = (R*)(lds + a.lds_pay_off);
 
+  constexpr int NP = kPair ? 2 : 1;
+  const int64_t n_own = kPair ? a.n_paths / 2 : a.n_paths;
   const int64_t path = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const bool active = path < a.n_paths;
-  const int64_t pc = active ? path : a.n_paths - 1;
+  const bool active = path < n_own;
+  const int64_t pc = active ? path : n_own - 1;
 
   // Local-vol table: stage in LDS when small.
   const R* tab = a.lv_vol;
@@ -324,11 +330,16 @@ euler_kernel(EulerArgs<R> a) {
     __syncthreads();
   }
 
-  R x[D];
+  R xs[NP][D];
+  R* const x = xs[0];
 #pragma unroll
-  for (int c = 0; c < D; ++c) x[c] = a.x0[pc * a.x0_stride + c];
+  for (int q = 0; q < NP; ++q)
+#pragma unroll
+    for (int c = 0; c < D; ++c)
+      xs[q][c] = a.x0[(pc + q * n_own) * a.x0_stride + c];
 
-  Normals<R, RNG> nrm;
+  // the pair's first path is its own stream's: the plain counter
+  Normals<R, kPair ? (int)TQF_RNG_PHILOX : RNG> nrm;
   nrm.init(a.rng, pc, D, lds, a.n_steps);
 
   // path-major staging (block-uniform bookkeeping, flushed at the uniform
@@ -386,7 +397,10 @@ euler_kernel(EulerArgs<R> a) {
     if constexpr (kStage)
       put(a.init_slot, off);
     else
-      record<R, MODEL>(a, lds_pay, a.init_slot, x, off, path, active);
+#pragma unroll
+      for (int q = 0; q < NP; ++q)
+        record<R, MODEL>(a, lds_pay, a.init_slot, xs[q], off, path + q * n_own,
+                         active);
   }
 
   int lv_row = 0;
@@ -444,12 +458,22 @@ euler_kernel(EulerArgs<R> a) {
       }
       Stepper<R, MODEL>::step(a, x, zc, dt, sdt, tab, lv_row, lv_w, i, row,
                               pv);
+      if constexpr (kPair) {
+        R zm[D];
+#pragma unroll
+        for (int k = 0; k < D; ++k) zm[k] = -zc[k];
+        Stepper<R, MODEL>::step(a, xs[NP - 1], zm, dt, sdt, tab, lv_row, lv_w,
+                                i, row, pv);
+      }
       if (s >= 0) {
         const R off = kHasStepRow<MODEL> ? row.c[3] : (R)0;
         if constexpr (kStage)
           put(s, off);
         else
-          record<R, MODEL>(a, lds_pay, s, x, off, path, active);
+#pragma unroll
+          for (int q = 0; q < NP; ++q)
+            record<R, MODEL>(a, lds_pay, s, xs[q], off, path + q * n_own,
+                             active);
       }
     };
     // two steps per iteration with the normals alternating between zA and
@@ -629,7 +653,17 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   lds += pay;
   if (lds == 0) lds = 16;
 
-  const unsigned n_blocks = (unsigned)((n_paths + kBlock - 1) / kBlock);
+  // Antithetic records on coalesced rows: both mirrors in one thread, the
+  // normals (in float64 most of the step) drawn once.  float64 Brownian
+  // paths, 100 records: 386 -> 264 us at 2^20 paths (839 MB), 127 -> 89 at
+  // 2^18, 76 -> 71 at 2^16; float32 139 -> 107 at 2^20.  Below 2^16 paths
+  // half the threads leave SIMDs empty and nothing is gained (69 and 71 us
+  // at 2^14).  Path-major records stage 64 consecutive paths a wave, and
+  // payoff sums keep their order, so both stay one path to a thread.
+  const bool pair = rng_kind == TQF_RNG_PHILOX_ANTITHETIC &&
+                    a.mode == TQF_OUT_STEP_MAJOR && n_paths >= kPairMinPaths;
+  const int64_t n_thr = pair ? n_paths / 2 : n_paths;
+  const unsigned n_blocks = (unsigned)((n_thr + kBlock - 1) / kBlock);
   void (*kern)(EulerArgs<R>) = nullptr;
   const int kind = (m->kind == TQF_MODEL_HESTON_FT && m->p[5] != 0.0)
                        ? kModelHestonOwn
@@ -656,6 +690,17 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   TQF_PICK_RNG(TQF_MODEL_HULL_WHITE)
 #undef TQF_PICK_RNG
 #undef TQF_PICK
+#define TQF_PICK_PAIR(MODEL) \
+  if (pair && kind == MODEL) \
+    kern = euler_kernel<R, MODEL, TQF_RNG_PHILOX_ANTITHETIC, false, true>;
+  TQF_PICK_PAIR(TQF_MODEL_GBM)
+  TQF_PICK_PAIR(TQF_MODEL_CONST)
+  TQF_PICK_PAIR(TQF_MODEL_HESTON_FT)
+  TQF_PICK_PAIR(kModelHestonOwn)
+  TQF_PICK_PAIR(TQF_MODEL_LOCAL_VOL)
+  TQF_PICK_PAIR(TQF_MODEL_HESTON_QE)
+  TQF_PICK_PAIR(TQF_MODEL_HULL_WHITE)
+#undef TQF_PICK_PAIR
   if (!kern) return set_error(TQF_ENOTIMPL, "unsupported model/rng combination");
   hipLaunchKernelGGL(kern, dim3(n_blocks), dim3(kBlock), lds, stream, a);
   int rc = check_launch("tqf_euler");
