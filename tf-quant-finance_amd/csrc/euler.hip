@@ -629,7 +629,8 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   a.x0_stride = x0_stride;
 
   // dynamic LDS: Sobol high-bit words | local-vol table | payoff sums and
-  // spot rows; the float32 inverse-CDF table is static LDS (kIcdfLdsBytes)
+  // spot rows; the float32 inverse-CDF tables are static LDS (at most
+  // kDyadicLdsBytes)
   size_t pay = 0;
   const bool stage = a.mode == TQF_OUT_PATH_MAJOR;
   a.stage_recs = kStageWords / D;

@@ -1041,7 +1041,8 @@ bool moment_plan(int d, int deg, int n_pairs, MomentPlan* out) {
 // column steps took 41, the trailing updates 33, the back solve 25 (each left
 // out in turn).  Row broadcasts in place of LDS-crossbar shuffles, rows above
 // the pivot skipped at compile time, the factored tile kept out of the
-// register tiles and all tile loads issued together: 131 us.
+// register tiles and all tile loads issued together: 133 us (only for tiles
+// that exist: with loads for all 17 a K = 9 solve took 4 us longer).
 constexpr int kSolveWaves = 8;
 constexpr int kSolveThreads = 64 * kSolveWaves;
 constexpr int kBT = 16;         // tile edge
@@ -1148,22 +1149,25 @@ lsm_solve_kernel(const double* __restrict__ g, int K, double rtol,
 #pragma unroll
   for (int q = 0; q < kBTiles; ++q) {
     const int a = tile_a(q), b = tile_b(q);
+    tile[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+    if (a >= 0)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
-      tile[q][r] = g[a >= 0 && row < n && col < n ? row * kext + col : 0];
-    }
+      for (int r = 0; r < 4; ++r) {
+        const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
+        tile[q][r] = g[row < n && col < n ? row * kext + col : 0];
+      }
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < kBTiles; ++q) {
     const int a = tile_a(q), b = tile_b(q);
+    if (a >= 0)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
-      tile[q][r] = a >= 0 && row < n && col < n
-                       ? tile[q][r] * (dsc[row] * dsc[col]) : 0.0;
-    }
+      for (int r = 0; r < 4; ++r) {
+        const int row = kBT * a + rl + 4 * r, col = kBT * b + cl;
+        tile[q][r] = row < n && col < n
+                         ? tile[q][r] * (dsc[row] * dsc[col]) : 0.0;
+      }
     __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
