@@ -1041,7 +1041,7 @@ bool moment_plan(int d, int deg, int n_pairs, MomentPlan* out) {
 // column steps took 41, the trailing updates 33, the back solve 25 (each left
 // out in turn).  Row broadcasts in place of LDS-crossbar shuffles, rows above
 // the pivot skipped at compile time, the factored tile kept out of the
-// register tiles and all tile loads issued together: 133 us (only for tiles
+// register tiles and all tile loads issued together: 134 us (only for tiles
 // that exist: with loads for all 17 a K = 9 solve took 4 us longer).
 constexpr int kSolveWaves = 8;
 constexpr int kSolveThreads = 64 * kSolveWaves;
