@@ -495,3 +495,34 @@ def test_shared_paths_exponential_and_monomial_mask():
   np.testing.assert_allclose(_np(v[0]), np.where(first > cont, first, last),
                              rtol=1e-15)
   assert int(ranks[0, 0]) == 1
+
+
+@pytest.mark.parametrize('n_ex', [1, 2])
+def test_one_asset_table_payoff_keeps_the_last_dates_values(n_ex):
+  # the value at the last date is the table's own, negative or not a number
+  # (as with several assets); before it such an entry is never exercised
+  n = 512
+  g = torch.Generator(device='cuda').manual_seed(5)
+  x = 100 + torch.randn((n, n_ex, 1), dtype=torch.float64, device='cuda',
+                        generator=g)
+  tab = 0.5 * (x[:, None, :, 0] - 100.0)  # [N, 1, n_ex], half of it negative
+  df = np.full(n_ex, 0.97)**np.arange(1, n_ex + 1)
+  basis = lsm.make_polynomial_basis(2)
+  price = lambda p, t: float(_np(lsm.least_square_mc(
+      p, list(range(n_ex)), lsm.make_table_payoff(t), basis,
+      discount_factors=df))[0])
+  # a second asset that never moves adds nothing to the regression
+  two = torch.cat([x, torch.full_like(x, 100.0)], -1)
+  want = price(two, tab)
+  assert abs(price(x, tab) - want) <= 1e-10 * abs(want)
+  if n_ex == 1:
+    assert abs(want - 0.97 * float(tab.mean())) <= 1e-12
+  else:
+    early = tab.clone()
+    early[7, 0, 0] = float('nan')
+    want = price(two, early)
+    assert np.isfinite(want)
+    assert abs(price(x, early) - want) <= 1e-10 * abs(want)
+  # on a path that is out of the money before, so it is held to the end
+  tab[int(torch.argmin(x[:, 0, 0])), 0, -1] = float('nan')
+  assert np.isnan(price(two, tab)) and np.isnan(price(x, tab))

@@ -88,12 +88,14 @@ __device__ __forceinline__ bool in_money(const PassItem& it, double x,
   return it.payoff == TQF_PAYOFF_BASKET_PUT ? x < it.strike : x > it.strike;
 }
 
-// The payoff of a path in the money, else 0.
+// The payoff of a path in the money, else 0; a table's own value (the last
+// date keeps it whatever its sign, or NaN; no continuation is below 0, so a
+// date before it never exercises one that is not positive).
 template <int LOGM>
 __device__ __forceinline__ double payoff(const PassItem& it, double x,
                                          double shift, const double* tab,
                                          int64_t p) {
-  if (it.payoff == TQF_PAYOFF_TABLE) return tab[p] > 0 ? tab[p] : 0.0;
+  if (it.payoff == TQF_PAYOFF_TABLE) return tab[p];
   if (!in_money<LOGM>(it, x, shift, tab, p)) return 0.0;
   const double s = LOGM == 2 ? exp_f64(fma(it.scale, x, shift)) : x;
   const double v = it.payoff == TQF_PAYOFF_BASKET_PUT ? it.strike - s
