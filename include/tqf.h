@@ -462,7 +462,8 @@ typedef struct tqf_swaption_plan {
  * the regression's inputs, float64 and date-major: short_rate [n_ex][n],
  * payoff [n_payoffs][n_ex][n], discounts [n_ex + 1][n] (row 0 = 1, row u + 1
  * = exp(-sum of r dt up to exercise date u)).  Every exercise index must
- * have its date: rows without one are not written. */
+ * have its date: rows without one are not written.  NaN values stay NaN, and
+ * row 1 of discounts is NaN for a path with a rate that is not finite. */
 int tqf_swaption_inputs(const void* rates, int64_t stride_path,
                         int64_t stride_time, int64_t n_paths, int32_t dtype,
                         const tqf_swaption_plan* plan, double* short_rate,

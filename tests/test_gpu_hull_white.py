@@ -257,3 +257,51 @@ def test_swaption_inputs_kernel_matches_the_tensor_operations(n, dtype):
     if n > 4:  # a handful of rows fits every path: no stable regression
       np.testing.assert_allclose(got, want, rtol=tol)
     assert np.all(np.isfinite(got))
+
+
+@pytest.mark.parametrize('what', ['volatility', 'curve', 'far_curve', 'path'])
+def test_nan_market_data_gives_a_nan_price(what):
+  # what the tensor operations give: a bond constant or a rate that is not a
+  # number reaches every price (their products run over all bonds and dates)
+  nan = float('nan')
+  ex = np.array([[1.0, 1.5, 2.0], [1.5, 2.0, 2.0]])
+  end = np.clip(ex[..., None] + np.array([0.5, 1.0]), 0.0, 2.5)
+  dcf, cpn = 0.5 * np.ones_like(end), 0.011 * np.ones_like(end)
+  last = {'curve': -1.0, 'far_curve': 2.2}.get(what, 9.0)
+  curve = lambda t: torch.where(torch.as_tensor(t) <= last, 0.01, nan).to(
+      torch.float64)
+  vol = nan if what == 'volatility' else 0.01
+  model = tqf.models.hull_white.HullWhiteModel1F(0.03, vol, curve,
+                                                 dtype=torch.float64)
+  plan = sw._plan(ex, end, 0.25)
+  rates = model.sample_paths(plan['sim_times'], num_samples=512,
+                             random_type=RandomType.STATELESS, seed=[3, 1])
+  if what == 'path':
+    rates[77, 5] = nan
+  basis = tqf.models.longstaff_schwartz.make_polynomial_basis(2)
+  want = _np(sw._price_on_paths(
+      plan, sw._exercise_bonds(model, plan, rates, end), rates, end, dcf, cpn,
+      basis, torch.float64))
+  got = _np(sw._price_native(model, plan, rates, end, dcf, cpn, 2,
+                             torch.float64))
+  assert np.all(np.isnan(want)) and np.all(np.isnan(got))
+
+
+def test_nan_coupon_stays_with_its_swaption():
+  ex = np.array([[1.0, 1.5], [1.0, 1.5]])
+  end = ex[..., None] + np.array([0.5, 1.0])
+  dcf, cpn = 0.5 * np.ones_like(end), 0.011 * np.ones_like(end)
+  cpn[1] = np.nan
+  model = tqf.models.hull_white.HullWhiteModel1F(0.03, 0.01, _flat,
+                                                 dtype=torch.float64)
+  plan = sw._plan(ex, end, 0.25)
+  rates = model.sample_paths(plan['sim_times'], num_samples=512,
+                             random_type=RandomType.STATELESS, seed=[3, 1])
+  basis = tqf.models.longstaff_schwartz.make_polynomial_basis(2)
+  want = _np(sw._price_on_paths(
+      plan, sw._exercise_bonds(model, plan, rates, end), rates, end, dcf, cpn,
+      basis, torch.float64))
+  got = _np(sw._price_native(model, plan, rates, end, dcf, cpn, 2,
+                             torch.float64))
+  assert np.isnan(want[1]) and np.isnan(got[1])
+  np.testing.assert_allclose(got[0], want[0], rtol=1e-11)

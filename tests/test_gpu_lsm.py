@@ -526,3 +526,17 @@ def test_one_asset_table_payoff_keeps_the_last_dates_values(n_ex):
   # on a path that is out of the money before, so it is held to the end
   tab[int(torch.argmin(x[:, 0, 0])), 0, -1] = float('nan')
   assert np.isnan(price(two, tab)) and np.isnan(price(x, tab))
+
+
+def test_shared_paths_exponential_at_its_ends():
+  # the payoff of a zero-strike call on log prices is exp itself: 0 far below
+  # the subnormals, one unit of them within, infinity above the range
+  x = torch.tensor([-np.inf, -1e300, -1e4, -746.5, -745.2, -745.1, -744.0,
+                    -708.5, 709.7, 709.9, 710.5, 1e300, np.inf],
+                   dtype=torch.float64, device='cuda')
+  it = {'payoff': lsm.PAYOFF_MAX_CALL, 'strike': 0.0, 'df': np.ones(2)}
+  v, _, _ = lsm.price_shared(x.reshape(-1, 1), [0], [it], 2, 7, None,
+                             x.device, basis_log=2)
+  with np.errstate(over='ignore', under='ignore'):
+    want = np.exp(_np(x))
+  np.testing.assert_allclose(_np(v[0]), want, rtol=4.5e-16, atol=5e-324)

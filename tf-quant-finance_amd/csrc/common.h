@@ -187,19 +187,23 @@ __device__ __forceinline__ T ld_uniform(const T* p, int64_t i) {
   return ((const __attribute__((address_space(4))) T*)p)[i];
 }
 
-// exp(x): 2^n e^r with r = x - n ln 2 (two-part ln 2) and the Taylor sum of
-// e^r to r^13 (|r| <= 0.347: remainder 5e-18).  The coefficients come through
-// scalar loads and enter the FMAs as scalar operands: 20 float64
+// exp(x): 2^n e^r with r = x - n ln 2 (ln 2 in the two parts published with
+// Sun's fdlibm: the product of n and the first is exact) and the Taylor sum
+// of e^r to r^13 (|r| <= 0.347: remainder 5e-18).  The coefficients come
+// through scalar loads and enter the FMAs as scalar operands: 22 float64
 // instructions, where the math library's function takes 47 instructions with
-// its coefficients moved into vector registers at every call.
+// its coefficients moved into vector registers at every call.  0 below -746,
+// infinity from 709.79 on (x itself stays in r, so an infinite x reaches the
+// sum), NaN for NaN: the comparison is false for it, where fmax would return
+// its other operand.
 static __constant__ double kExpCoef[12] = {
     1.0 / 6227020800.0, 1.0 / 479001600.0, 1.0 / 39916800.0, 1.0 / 3628800.0,
     1.0 / 362880.0,     1.0 / 40320.0,     1.0 / 5040.0,     1.0 / 720.0,
     1.0 / 120.0,        1.0 / 24.0,        1.0 / 6.0,        0.5};
 
 __device__ __forceinline__ double exp_f64(double x) {
-  x = fmin(fmax(x, -745.0), 710.0);
-  const double n = __builtin_rint(x * 1.4426950408889634);
+  x = x < -746.0 ? -746.0 : x;
+  const double n = __builtin_rint(fmin(x, 710.0) * 1.4426950408889634);
   double r = fma(n, -6.93147180369123816490e-01, x);
   r = fma(n, -1.90821492927058770002e-10, r);
   double p = ld_uniform(kExpCoef, 0);

@@ -12,7 +12,7 @@
 // date-major layout.  As separate tensor operations (gathers, a matrix
 // product for the discounts, an exponential over [N, batch, dates, payments]
 // and a product with block-diagonal weights) the same took about 2 ms for
-// two swaptions of 2^19 paths; bound by the exponentials here (20 float64
+// two swaptions of 2^19 paths; bound by the exponentials here (22 float64
 // instructions each).
 #include "common.h"
 
@@ -57,11 +57,16 @@ swaption_inputs_kernel(const R* __restrict__ rates, SwaptionArgs a) {
         v = fma(-ld_uniform(a.entries, 3 * (int64_t)k + 2),
                 exp_f64(fma(-r, ld_uniform(a.entries, 3 * (int64_t)k + 1),
                             ld_uniform(a.entries, 3 * (int64_t)k))), v);
-      // a date without entries is not one of the swaption's own
+      // a date without entries is not one of the swaption's own; NaN stays
       a.payoff[((int64_t)b * a.n_ex + u) * a.n + p] =
-          k1 > k0 && v > 0 ? v : 0.0;
+          k1 == k0 || v < 0 ? 0.0 : v;
     }
   }
+  // a path whose rates are not finite has no price: its values at dates
+  // before the first such rate may look sound, and its sums of the
+  // regression are NaN, so its last factor, which every value is multiplied
+  // by, says so
+  if (!(total - total == 0.0)) a.discounts[a.n + p] = total - total;
 }
 
 }  // namespace

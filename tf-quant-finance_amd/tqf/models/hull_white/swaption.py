@@ -117,9 +117,12 @@ def _plan(ex, pay, time_step):
 
 
 def _payoff_entries(model, plan, pay, dcf, cpn):
-  """(first [n_u * B + 1], entries [., 3]) of tqf_swaption_inputs: per
+  """(first [n_u * B + 1], entries [., 3], sound) of tqf_swaption_inputs: per
   exercise date of the union and swaption, the constants (C, G) of its
-  payment dates' bonds P = exp(C - r G) and their weights."""
+  payment dates' bonds P = exp(C - r G) and their weights.  sound: every bond
+  is a number.  One that is not makes every price NaN, also with a zero
+  weight (which leaves its bond out of the entries): so do the tensor
+  operations, whose products run over all bonds."""
   shape = np.broadcast_shapes(pay.shape, plan['ex_full'].shape)
   n_ex, n_pay = shape[-2:]
   flat_b = int(np.prod(plan['batch_shape'])) if plan['batch_shape'] else 1
@@ -145,8 +148,9 @@ def _payoff_entries(model, plan, pay, dcf, cpn):
         # a swap with no payment left still has its own date
         entries += own_entries or [(0.0, 0.0, 0.0)]
       first.append(len(entries))
+  sound = not (np.isnan(c).any() or np.isnan(g).any() or np.isposinf(c).any())
   return (np.asarray(first, np.int32),
-          np.asarray(entries, np.float64).reshape(-1, 3))
+          np.asarray(entries, np.float64).reshape(-1, 3), sound)
 
 
 def _price_native(model, plan, r_t, pay, dcf, cpn, degree, tdt):
@@ -159,7 +163,9 @@ def _price_native(model, plan, r_t, pay, dcf, cpn, degree, tdt):
   flat_b = int(np.prod(plan['batch_shape'])) if plan['batch_shape'] else 1
   slot = np.full(sim_times.shape[0], -1, np.int32)
   slot[np.searchsorted(sim_times, unique_ex)] = np.arange(n_u)
-  first, entries = _payoff_entries(model, plan, pay, dcf, cpn)
+  first, entries, sound = _payoff_entries(model, plan, pay, dcf, cpn)
+  if not sound:
+    return torch.full((flat_b,), float('nan'), dtype=tdt, device=dev)
   pl = _native.SwaptionPlan()
   pl.n_dates, pl.n_ex, pl.n_payoffs = sim_times.shape[0], n_u, flat_b
   keep = []
