@@ -487,3 +487,16 @@ def test_parameter_values_read_together(dtypes, shapes):
             for v, dt, sh in zip(vals, dtypes, shapes)]
   got = differentiable._values(params)
   assert got == [float(p.detach().cpu().reshape(())) for p in params]
+
+
+@pytest.mark.parametrize('greeks', ['tangent', 'adjoint'])
+@pytest.mark.parametrize('field', ['rate', 's0', 'maturity'])
+def test_batch_nan_input_gives_a_nan_price(field, greeks):
+  cs = [_gbm(0, paths=256, steps=5), _heston(1, paths=256, steps=5)]
+  bad = [dict(c, **{field: float('nan')}) for c in cs]
+  plan = batch_lib.BatchPlan(bad + cs, tile=64, greeks=greeks)
+  plan.launch()
+  res = plan.results()
+  assert all(np.isnan(r['price'][0]) and np.isnan(r['delta'][0])
+             for r in res[:2])
+  assert all(np.isfinite(v[0]) for r in res[2:] for v in r.values())

@@ -158,8 +158,9 @@ __device__ __forceinline__ void heston_payoff(const Contract& c, float x,
   const float disc = __expf(-c.r * c.t);
   // one rounding of S - K, whatever the caller contracts
   const float gain = fma_r(c.s0, e, -c.strike);
-  pay = gain > 0.f ? disc * gain : 0.f;
-  xb = gain > 0.f ? disc * (c.s0 * e) : 0.f;
+  // NaN compares false and stays
+  pay = gain <= 0.f ? 0.f : disc * gain;
+  xb = gain <= 0.f ? 0.f : disc * (c.s0 * e);
 }
 
 // One Heston path with the checkpointed reverse sweep.  ck: this thread's
