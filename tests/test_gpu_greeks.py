@@ -500,3 +500,21 @@ def test_batch_nan_input_gives_a_nan_price(field, greeks):
   assert all(np.isnan(r['price'][0]) and np.isnan(r['delta'][0])
              for r in res[:2])
   assert all(np.isfinite(v[0]) for r in res[2:] for v in r.values())
+
+
+def test_batch_tangents_at_a_subnormal_variance():
+  # the hardware root of a subnormal variance is 0: no 1 / sqrt(v) term, as
+  # in the reverse sweep
+  cs = [_heston(i, steps=40, paths=512, v0=v0, theta=0.0, xi=xi, kappa=1.5)
+        for i, (v0, xi) in enumerate([(1e-40, 0.0), (1e-39, 0.2),
+                                      (0.0, 0.2)])]
+  out = []
+  for greeks in ('tangent', 'adjoint'):
+    plan = batch_lib.BatchPlan(cs, tile=64, greeks=greeks)
+    plan.launch()
+    out.append(plan.results())
+  for c, t, a in zip(cs, *out):
+    for name in t:
+      assert np.isfinite(t[name]).all(), (c['v0'], name, t[name])
+      assert abs(t[name][0] - a[name][0]) <= 1e-3 * abs(a[name][0]) + 1e-6, (
+          c['v0'], name, t[name], a[name])

@@ -279,8 +279,9 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
     const float dw0 = heston_dw(k, z0), dw1 = heston_dw(k, z1);
     const float cu = fma_r(k.s1r, dw1, k.rho * dw0);
     // d sqrt(v+) / dv+ by the hardware reciprocal (one instruction in
-    // place of a correctly rounded division by sq)
-    const float h = 0.5f * __builtin_amdgcn_rcpf(sq);
+    // place of a correctly rounded division by sq); 0 where the root is, as
+    // in the reverse sweep (the hardware root of a subnormal v is 0)
+    const float h = sq > 0.f ? 0.5f * __builtin_amdgcn_rcpf(sq) : 0.f;
     const float a = pos ? fma_r(h, dw0, k.mdt2) : 0.f;
     const float b = pos ? fma_r(h * k.xi, cu, b0) : 1.f;
 #pragma unroll
