@@ -518,3 +518,31 @@ def test_batch_tangents_at_a_subnormal_variance():
       assert np.isfinite(t[name]).all(), (c['v0'], name, t[name])
       assert abs(t[name][0] - a[name][0]) <= 1e-3 * abs(a[name][0]) + 1e-6, (
           c['v0'], name, t[name], a[name])
+
+
+def test_batch_tangents_keep_the_digits_of_small_steps():
+  # 500 steps of dt kappa about 1e-4, v far from 0 (its total noise is
+  # 0.006 around 0.09).  A factor 1 - dt kappa held as one float32 repeats
+  # its rounding (up to 3e-8) in every step: up to 1.5e-5 of d/dv0.  As an
+  # increment, a step adds one rounding of the tangent (at most 6e-8), which
+  # differs from step to step and path to path: sqrt(500) 6e-8 / sqrt(3) =
+  # 8e-7 a path, its mean over the paths below; the constants' own roundings
+  # come in by dt kappa times 500 steps, 6e-8 of kappa T.  Hence 1e-6 of the
+  # terms' root mean square
+  cs = [_heston(i, steps=500, paths=4096, t=0.05, v0=0.09, xi=0.1,
+                theta=0.09, kappa=k)
+        for i, k in enumerate([0.7, 1.1, 1.3, 1.7, 1.9, 2.3])]
+  plan = batch_lib.BatchPlan(cs, tile=256, seed=9, greeks='tangent')
+  plan.launch()
+  for c, r in zip(cs, plan.results()):
+    n, m = c['n_steps'], c['n_paths']
+    z = orng.normals(m, 2 * n, 9, stream=c['stream_id'],
+                     dtype=np.float32).astype(np.float64).reshape(m, n, 2)
+    want, se = oheston.ft_euler_call_greeks(
+        np.log(c['s0']), c['v0'], c['kappa'], c['theta'], c['xi'], c['rho'],
+        c['rate'], c['strike'], np.linspace(0.0, c['maturity'], n + 1), z)
+    rms = np.sqrt(want**2 + m * se**2)
+    q = batch_lib.GREEK_NAMES[c['kind']].index('dv0')
+    err = abs(r['dv0'][0] - want[q]) / rms[q]
+    print(c['kappa'], 'd/dv0 error', err, flush=True)
+    assert err <= 1e-6

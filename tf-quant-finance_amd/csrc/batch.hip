@@ -249,15 +249,19 @@ __device__ void heston_path(const Contract& c, int64_t p, uint32_t stream,
 // sweep above, with the same subgradient 0 at v <= 0: the price depends on
 // x_T only, so each Greek is x-bar ("xb" below) times the x-tangent, and
 // delta and rho are closed form as in the reverse sweep.
-//   x'  <- x' + A v',  A = -dt/2 + h dw0            (0 where v <= 0)
-//   v'  <- B v' + dv'/dp,  B = 1 - dt kappa + h xi cu  (1 where v <= 0)
-// with h = 1 / (2 sqrt v) and cu = rho dw0 + s dw1.  A and B are the same
-// for the five tangents, so each costs two FMAs (a select, a product and
-// four FMAs when the factors are applied one by one).  Bound by VALU issue:
-// 69 instructions and 233 cycles a step and wave, of which half a Philox
-// block is 66 and the Box-Muller pair 62; five waves per SIMD (the launch
-// bound keeps it at 96 registers).  A book of 256 contracts (8.3e9 GBM and
-// 8.3e9 Heston path-steps) takes 4.40 ms, 5.68 ms before.
+//   x'  <- x' + A v',  A = -dt/2 + h dw0
+//   v'  <- v' + (B v' + dv'/dp),  B = -dt kappa + h xi cu
+// with h = 1 / (2 sqrt v) and cu = rho dw0 + s dw1, A and B 0 where v <= 0.
+// They are the same for the five tangents, so a step is an FMA for x' and an
+// FMA and an addition for v' (a select, a product and four FMAs when the
+// factors are applied one by one).  B is the increment, not 1 + B: dt kappa
+// of 1e-3 would keep 14 bits beside the 1, with the same rounding in every
+// step (median error of d/dv0 over a book 1.4e-6, as an increment 1.2e-7).
+// Bound by VALU issue: 75 instructions and about 250 cycles a step and wave,
+// of which half a Philox block is 66 and the Box-Muller pair 62; five waves
+// per SIMD (the launch bound keeps it at 96 registers).  A book of 256
+// contracts (8.3e9 GBM and 8.3e9 Heston path-steps) takes 4.47 ms, 5.47 with
+// the factors applied one by one, 4.28 with 1 + B.
 __device__ void heston_path_tangent(const Contract& c, int64_t p,
                                     uint32_t stream,
                                     const PhiloxKeys<true>& keys, float* g) {
@@ -266,7 +270,6 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
   const double dt = (double)c.t / n;
   const float drho_s = -c.rho / k.s1r;  // d sqrt(1-rho^2) / d rho
   const float mdt = (float)-dt;
-  const float b0 = (float)(1.0 - dt * c.kappa);
   const uint32_t plo = (uint32_t)p, phi = (uint32_t)(p >> 32);
   float x = 0.f, v = c.v0;
   // tangents of (x, v) for v0, kappa, theta, xi, rho
@@ -283,14 +286,14 @@ __device__ void heston_path_tangent(const Contract& c, int64_t p,
     // in the reverse sweep (the hardware root of a subnormal v is 0)
     const float h = sq > 0.f ? 0.5f * __builtin_amdgcn_rcpf(sq) : 0.f;
     const float a = pos ? fma_r(h, dw0, k.mdt2) : 0.f;
-    const float b = pos ? fma_r(h * k.xi, cu, b0) : 1.f;
+    const float b = pos ? fma_r(h * k.xi, cu, k.mdtk) : 0.f;
 #pragma unroll
     for (int q = 0; q < 5; ++q) tx[q] = fma_r(a, tv[q], tx[q]);
-    tv[0] *= b;
-    tv[1] = fma_r(mdt, vp - k.theta, b * tv[1]);                 // kappa
-    tv[2] = fma_r(b, tv[2], -k.mdtk);                            // theta
-    tv[3] = fma_r(b, tv[3], sq * cu);                            // xi
-    tv[4] = fma_r(b, tv[4], (k.xi * sq) * fma_r(drho_s, dw1, dw0));  // rho
+    tv[0] = fma_r(b, tv[0], tv[0]);
+    tv[1] += fma_r(b, tv[1], mdt * (vp - k.theta));               // kappa
+    tv[2] += fma_r(b, tv[2], -k.mdtk);                            // theta
+    tv[3] += fma_r(b, tv[3], sq * cu);                            // xi
+    tv[4] += fma_r(b, tv[4], (k.xi * sq) * fma_r(drho_s, dw1, dw0));  // rho
     // the state update of the reverse-mode path, so both modes price the
     // same paths bit for bit
     heston_step(k, vp, sq, dw0, cu, x, v);
