@@ -540,3 +540,33 @@ def test_shared_paths_exponential_at_its_ends():
   with np.errstate(over='ignore', under='ignore'):
     want = np.exp(_np(x))
   np.testing.assert_allclose(_np(v[0]), want, rtol=4.5e-16, atol=5e-324)
+
+
+@pytest.mark.parametrize('table', [False, True])
+def test_many_payoffs_of_one_asset_need_the_memory_of_one_group(table):
+  # 160 payoffs on 2^16 paths: the value columns (and the transposed tables)
+  # of one group of payoffs are held, not those of every payoff
+  n, b, n_ex = 2**16, 160, 2
+  x = 100 + torch.randn((n, n_ex, 1), dtype=torch.float64, device='cuda')
+  strikes = np.linspace(95.0, 105.0, b)
+  basis = lsm.make_polynomial_basis(2)
+  if table:
+    k = torch.as_tensor(strikes, device='cuda')
+    pay = lsm.make_table_payoff(
+        torch.relu(k[None, :, None] - x[:, None, :, 0]))
+  else:
+    pay = lsm.make_basket_put_payoff(strikes, dtype=torch.float64)
+  df = np.array([0.99, 0.98])
+  torch.cuda.synchronize()
+  torch.cuda.reset_peak_memory_stats()
+  before = torch.cuda.memory_allocated()
+  got = _np(lsm.least_square_mc(x, [0, 1], pay, basis, discount_factors=df))
+  extra = torch.cuda.max_memory_allocated() - before
+  column = 8 * n
+  # 16 columns, their two-date tables, the step-major copy of the paths and
+  # the per-workgroup rows (below eight columns)
+  assert extra <= column * (16 * (1 + n_ex * table) + n_ex + 8)
+  want = [float(_np(lsm.least_square_mc(
+      x, [0, 1], lsm.make_basket_put_payoff([s], dtype=torch.float64), basis,
+      discount_factors=df))[0]) for s in strikes[[0, 15, 16, 159]]]
+  np.testing.assert_allclose(got[[0, 15, 16, 159]], want, rtol=1e-13)

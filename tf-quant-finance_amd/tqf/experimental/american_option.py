@@ -89,7 +89,7 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
                 'log_scale': scale(b)} for b in range(n_opt)]
       _, res, _ = lsm_lib.price_shared(
           w, ex, items, degree, (2 << degree) - 1, num_calibration_samples,
-          dev, basis_log=2)
+          dev, basis_log=2, keep_values=False)
       prices = res[:, 0].cpu().numpy()
     else:
       outs = []

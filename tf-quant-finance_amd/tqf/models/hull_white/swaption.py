@@ -190,7 +190,7 @@ def _price_native(model, plan, r_t, pay, dcf, cpn, degree, tdt):
             'df': np.ones(n_u + 1)} for b in range(flat_b)]
   _, res, _ = lsm.price_shared(rate.t(), list(range(n_u)), items, degree,
                                (2 << degree) - 1, None, dev,
-                               path_discounts=disc)
+                               path_discounts=disc, keep_values=False)
   return res[:, 0].to(tdt)
 
 

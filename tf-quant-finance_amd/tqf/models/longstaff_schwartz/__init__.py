@@ -175,6 +175,9 @@ def step_major_f64(paths):
 
 
 _SHARED_MAX_ITEMS, _SHARED_MAX_DEGREE = 16, 4
+# value columns and transposed tables held at once (a launch takes fewer than
+# _SHARED_MAX_ITEMS payoffs from 2^25 paths on): 1/72 of a card's memory
+_SHARED_BYTES = 4 << 30
 
 
 def shared_supported(dim, degree, n_paths, num_calib):
@@ -184,16 +187,19 @@ def shared_supported(dim, degree, n_paths, num_calib):
 
 
 def price_shared(paths, ex, items, degree, mask, num_calib, dev,
-                 basis_log=0, path_discounts=None):
-  """Prices several payoffs on the same one-asset paths, one launch per
-  exercise date for all of them (tqf_lsm_price_shared).
+                 basis_log=0, path_discounts=None, keep_values=True):
+  """Prices several payoffs on the same one-asset paths, a pass and a solve
+  per exercise date for all of them (tqf_lsm_price_shared).
 
   paths: float64 [N, T] with any strides.  items: dicts with payoff, strike,
-  df [n_ex + 1] (padded), and optionally table [T, N] (contiguous) or
-  log_shift [n_ex] and log_scale (basis_log 2: the log price at date e is
-  log_shift[e] + log_scale * stored value).  mask: bit m set when the
-  monomial of exponent m is in the basis.  Returns (values [B, N] at the
-  first exercise date, results [B, 2], ranks [B, max(n_ex - 1, 1)])."""
+  df [n_ex + 1] (padded), and optionally table [T, N] (contiguous, or a
+  function that makes it when its group of payoffs is launched) or log_shift
+  [n_ex] and log_scale (basis_log 2: the log price at date e is log_shift[e]
+  + log_scale * stored value).  mask: bit m set when the monomial of exponent
+  m is in the basis.  Returns (values [B, N] at the first exercise date,
+  results [B, 2], ranks [B, max(n_ex - 1, 1)]); without keep_values, values
+  holds the last group's payoffs only, so a long list of payoffs takes the
+  memory of one group."""
   n, nt = paths.shape
   l = _native.Lsm()
   l.paths = paths.data_ptr()
@@ -207,13 +213,18 @@ def price_shared(paths, ex, items, degree, mask, num_calib, dev,
     l.path_discounts = path_discounts.data_ptr()
   n_ex, nb = len(ex), len(items)
   exi = (ctypes.c_int32 * n_ex)(*ex)
-  values = torch.empty((nb, n), dtype=torch.float64, device=dev)
+  columns = 1 + (nt if any(callable(it.get('table')) for it in items) else 0)
+  group = max(1, min(_SHARED_MAX_ITEMS, nb, _SHARED_BYTES // (8 * n * columns)))
+  values = torch.empty((nb if keep_values else group, n), dtype=torch.float64,
+                       device=dev)
   results = torch.empty((nb, 2), dtype=torch.float64, device=dev)
   ranks = torch.empty((nb, max(n_ex - 1, 1)), dtype=torch.int32, device=dev)
   if n_ex < 2:
     ranks.zero_()
-  for b0 in range(0, nb, _SHARED_MAX_ITEMS):
-    part = items[b0:b0 + _SHARED_MAX_ITEMS]
+  out = values
+  for b0 in range(0, nb, group):
+    part = items[b0:b0 + group]
+    out = values[b0:] if keep_values else values[:len(part)]
     arr = (_native.LsmItem * len(part))()
     keep = []
     for o, it in zip(arr, part):
@@ -221,10 +232,12 @@ def price_shared(paths, ex, items, degree, mask, num_calib, dev,
       host = [np.ascontiguousarray(it['df'], np.float64)]
       o.df = host[0].ctypes.data
       if it.get('table') is not None:
-        o.payoff_table = it['table'].data_ptr()
+        table = it['table']() if callable(it['table']) else it['table']
+        host.append(table)
+        o.payoff_table = table.data_ptr()
       if it.get('log_shift') is not None:
         host.append(np.ascontiguousarray(it['log_shift'], np.float64))
-        o.log_shift = host[1].ctypes.data
+        o.log_shift = host[-1].ctypes.data
         o.log_scale = float(it['log_scale'])
       keep.append(host)
     ws = torch.empty(int(_native.lib().tqf_lsm_shared_workspace_size(
@@ -232,11 +245,11 @@ def price_shared(paths, ex, items, degree, mask, num_calib, dev,
     _native.call('tqf_lsm_price_shared', ctypes.byref(l), arr,
                  ctypes.c_int32(len(part)), ctypes.c_int32(mask), exi,
                  ctypes.c_int32(n_ex), ctypes.c_void_p(ws.data_ptr()),
-                 ctypes.c_void_p(values[b0].data_ptr()),
+                 ctypes.c_void_p(out.data_ptr()),
                  ctypes.c_void_p(results[b0].data_ptr()),
                  ctypes.c_void_p(ranks[b0].data_ptr()),
                  _native.stream_ptr(dev))
-  return values, results, ranks
+  return (values if keep_values else out), results, ranks
 
 
 def _native_lsm(x, ex, pspec, degree, df, num_calib, dtype, dev,
@@ -296,11 +309,13 @@ def _native_lsm(x, ex, pspec, degree, df, num_calib, dtype, dev,
             'strike': strikes[b if strikes.shape[0] > 1 else 0],
             'df': np.ones(df.shape[0]) if per_path else dfs[:, b]}
       if table is not None:
-        it['table'] = table[:, b if table.shape[1] > 1 else 0, :].T.contiguous()
+        it['table'] = lambda b=b: table[
+            :, b if table.shape[1] > 1 else 0, :].T.contiguous()
       items.append(it)
     mask = int(np.bitwise_or.reduce(1 << expo[:, 0].astype(np.int64)))
     values, res, ranks = price_shared(p64[:, :, 0], ex, items, degree, mask,
-                                      num_calib, dev, basis_log, pdb)
+                                      num_calib, dev, basis_log, pdb,
+                                      keep_values=False)
     if path_values is not None:
       path_values.copy_(values[-1])
     out = res[:, 0].to(dtype)
