@@ -570,3 +570,17 @@ def test_many_payoffs_of_one_asset_need_the_memory_of_one_group(table):
       x, [0, 1], lsm.make_basket_put_payoff([s], dtype=torch.float64), basis,
       discount_factors=df))[0]) for s in strikes[[0, 15, 16, 159]]]
   np.testing.assert_allclose(got[[0, 15, 16, 159]], want, rtol=1e-13)
+
+
+def test_american_options_without_an_option():
+  # a user basis prices option by option: none is an empty result; with the
+  # polynomial basis there is no launch to make
+  from tqf.experimental import american_option
+  price = lambda **kw: american_option.bs_lsm_price(
+      [], [1.0], [1.0], [0.2], [0.97], num_samples=64, num_exercise_times=3,
+      **kw)
+  user = lambda paths, t: torch.stack([torch.ones_like(paths[:, t, 0]),
+                                       paths[:, t, 0]])
+  assert price(basis_fn=user).shape == (0,)
+  with pytest.raises(ValueError, match='no option'):
+    price()

@@ -48,8 +48,6 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
   dev = _native.device()
   spots_np = np.asarray(utils.to_numpy(spots), np.float64).reshape(-1)
   n_opt = spots_np.shape[0]
-  if n_opt == 0:
-    raise ValueError('`spots` holds no option')
   expiry = _vec(expiry_times, n_opt, dtype)
   strike = _vec(strikes, n_opt, dtype) / spots_np
   vol = _vec(volatility, n_opt, dtype)
@@ -76,6 +74,8 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
     basis_fn = lsm_lib.make_polynomial_basis(2)
   bspec = getattr(basis_fn, '_tqf_basis', None)
   if bspec is not None and bspec[0] == 'poly':
+    if n_opt == 0:
+      raise ValueError('`spots` holds no option')
     degree = bspec[1]
     kind = lambda b: (lsm_lib.PAYOFF_MAX_CALL if call[b]
                       else lsm_lib.PAYOFF_BASKET_PUT)
