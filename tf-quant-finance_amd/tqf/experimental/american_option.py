@@ -31,6 +31,19 @@ from tqf.models import utils
 __all__ = ['bs_lsm_price']
 
 
+_STREAMS = {}
+_MAX_STREAMS = 4
+
+
+def _streams(dev, n):
+  """Up to _MAX_STREAMS side streams of `dev` (default priority), cached."""
+  key = str(dev)
+  pool = _STREAMS.setdefault(key, [])
+  while len(pool) < min(n, _MAX_STREAMS):
+    pool.append(torch.cuda.Stream(device=dev))
+  return pool[:min(n, _MAX_STREAMS)]
+
+
 def _vec(v, n, dtype):
   a = np.asarray(utils.to_numpy(v), np.float64).reshape(-1)
   return np.broadcast_to(a, [n]).astype(np.float64)
@@ -92,17 +105,30 @@ def bs_lsm_price(spots, expiry_times, strikes, volatility, discount_factors,
           dev, basis_log=2, keep_values=False)
       prices = res[:, 0].cpu().numpy()
     else:
+      # option by option, each of several on its own stream: the
+      # single-workgroup solves of one overlap the passes of the others (four
+      # options, degree 5, 2^18 paths and 20 dates: 4.3 ms, one after another
+      # 5.0; a single option takes 1.6 ms on a side stream and 1.4 here)
+      main = torch.cuda.current_stream(dev)
+      streams = _streams(dev, n_opt) if n_opt > 1 else [main]
       outs = []
       for b in range(n_opt):
-        log_s_t = torch.add(
-            torch.as_tensor(shift(b), device=dev).reshape(-1, 1), w_t,
-            alpha=scale(b))
-        # [N, T, 1] view of [T][1][N] memory
-        outs.append(lsm_lib._native_lsm(
-            log_s_t.unsqueeze(1).permute(2, 0, 1), ex,
-            (kind(b), np.array([strike[b]])), degree,
-            np.concatenate([[1.0], dfs(b)]).reshape(-1, 1, 1),
-            num_calibration_samples, torch.float64, dev, basis_log=2))
+        st = streams[b % len(streams)]
+        if st is not main:
+          st.wait_stream(main)  # the Brownian paths are the caller's
+        with torch.cuda.stream(st):
+          log_s_t = torch.add(
+              torch.as_tensor(shift(b), device=dev).reshape(-1, 1), w_t,
+              alpha=scale(b))
+          # [N, T, 1] view of [T][1][N] memory
+          outs.append(lsm_lib._native_lsm(
+              log_s_t.unsqueeze(1).permute(2, 0, 1), ex,
+              (kind(b), np.array([strike[b]])), degree,
+              np.concatenate([[1.0], dfs(b)]).reshape(-1, 1, 1),
+              num_calibration_samples, torch.float64, dev, basis_log=2))
+      for st in streams:
+        if st is not main:
+          main.wait_stream(st)
       prices = torch.cat(outs).cpu().numpy()
     return torch.as_tensor(prices * spots_np, dtype=dtype, device=dev)
   prices = []
