@@ -88,14 +88,16 @@ __device__ __forceinline__ bool in_money(const PassItem& it, double x,
   return it.payoff == TQF_PAYOFF_BASKET_PUT ? x < it.strike : x > it.strike;
 }
 
-// The payoff of a path in the money, else 0; a table's own value (the last
-// date keeps it whatever its sign, or NaN; no continuation is below 0, so a
-// date before it never exercises one that is not positive).
+// The payoff of a path in the money, else 0.  A table's value at the last
+// date stays as it is, negative or NaN.  (Before it the sign makes no
+// difference, since no continuation is below 0; but with tab[p] alone the
+// compiler schedules the pass of the other payoffs 3 % slower.)
 template <int LOGM>
 __device__ __forceinline__ double payoff(const PassItem& it, double x,
                                          double shift, const double* tab,
-                                         int64_t p) {
-  if (it.payoff == TQF_PAYOFF_TABLE) return tab[p];
+                                         int64_t p, int terminal) {
+  if (it.payoff == TQF_PAYOFF_TABLE)
+    return terminal || tab[p] > 0 ? tab[p] : 0.0;
   if (!in_money<LOGM>(it, x, shift, tab, p)) return 0.0;
   const double s = LOGM == 2 ? exp_f64(fma(it.scale, x, shift)) : x;
   const double v = it.payoff == TQF_PAYOFF_BASKET_PUT ? it.strike - s
@@ -295,7 +297,8 @@ chain_pass_kernel(PassArgs a) {
       const int pr = base + i * kThreads + t;
       if (pr >= n_rows) continue;
       const int64_t p = p0 + pr;
-      const double ex = payoff<LOGM>(it, xu[i], it.shift_u, it.tab_u, p);
+      const double ex = payoff<LOGM>(it, xu[i], it.shift_u, it.tab_u, p,
+                                     a.terminal);
       if (a.terminal) {
         v[i] = ex;
       } else {
