@@ -640,7 +640,7 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
     a.lds_spot_off = (int)((sums + 15) & ~(size_t)15);
     pay = (size_t)a.lds_spot_off + (size_t)kWaves * kWave * sizeof(R);
   }
-  const int rng_kind = kernel_rng<R>(r);
+  const int rng_kind = kernel_rng<R>(r, stage);
   size_t lds = (size_t)rng_lds_bytes(rng_kind, D);
   if (m->kind == TQF_MODEL_LOCAL_VOL) {
     const int64_t lv = (int64_t)m->lv_nt * m->lv_nx * (int64_t)sizeof(R);
@@ -680,7 +680,8 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   TQF_PICK(MODEL, TQF_RNG_SOBOL)                  \
   TQF_PICK(MODEL, TQF_RNG_SOBOL_SHIFTED)          \
   if constexpr (sizeof(R) == sizeof(float)) {     \
-    TQF_PICK(MODEL, kRngSobolDyadic)              \
+    if (kind == MODEL && rng_kind == kRngSobolDyadic) \
+      kern = euler_kernel<R, MODEL, kRngSobolDyadic, false>; \
   }
   TQF_PICK_RNG(TQF_MODEL_GBM)
   TQF_PICK_RNG(TQF_MODEL_CONST)

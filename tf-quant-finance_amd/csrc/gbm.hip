@@ -186,7 +186,7 @@ int launch(const tqf_gbm* g, const tqf_grid* grid, const tqf_rng* r,
   a.mode = mode;
   a.out = (R*)out;
   a.n_paths = n_paths;
-  const int rng_kind = kernel_rng<R>(r);
+  const int rng_kind = kernel_rng<R>(r, mode == TQF_OUT_PATH_MAJOR);
   size_t lds = ((size_t)rng_lds_bytes(rng_kind, g->dim) + 15) & ~(size_t)15;
   a.stage_off = (int)lds;
   a.stage_recs = kStageWords / g->dim;  // dim <= 16: at least 2

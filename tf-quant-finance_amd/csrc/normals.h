@@ -211,12 +211,15 @@ __device__ __forceinline__ float dyadic_f32(uint32_t v, int shl,
       __float_as_uint(z), s, k.sign, 0x78));
 }
 
-// The kernel's code for rng kind `kind`: the table transform where it
-// applies.
+// The kernel's code for a source of normals: the table transform where it
+// applies.  Not where path-major records are staged: their 34 KB a workgroup
+// let four share a CU, with the table's 8 KB three, which costs more than
+// erfinv_f32 (2^19 paths, 100 steps, 50 records: Heston 137 us against 152,
+// local volatility 179 against 225, Hull-White 100 against 125).
 template <typename R>
-inline int kernel_rng(const tqf_rng* r) {
+inline int kernel_rng(const tqf_rng* r, bool path_major) {
   return sizeof(R) == sizeof(float) && r->kind == TQF_RNG_SOBOL &&
-                 r->sobol_nd <= 24
+                 r->sobol_nd <= 24 && !path_major
              ? kRngSobolDyadic
              : r->kind;
 }
