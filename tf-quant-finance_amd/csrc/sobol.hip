@@ -388,39 +388,47 @@ sobol_points_run_kernel(const uint32_t* __restrict__ v, int dim, double scale,
             });
 }
 
-template <typename R>
+// The transform of a point, one kernel each: float32 reference points of at
+// most 24 digits take the table, of more erfinv_f32.  With the choice made in
+// the loop of one kernel every transform paid for the others' tables,
+// barrier and registers: 2^20 points of 16 dimensions 41.2 us (28.0 now, by
+// erfinv_f32 31.4), two dimensions of 2^22 points beyond 24 digits 45 (33.7),
+// float64 64 dimensions of 2^19 points 345 (307).
+enum NormalTransform { kRefErfinv, kRefTable, kShifted };
+
+template <typename R, int T>
 __global__ void __launch_bounds__(256)
 sobol_normals_run_kernel(const uint32_t* __restrict__ v, int dim, R scale,
                          int shl, int64_t n, int64_t first,
-                         const uint32_t* __restrict__ shift, int mode,
+                         const uint32_t* __restrict__ shift,
                          R* __restrict__ out, int dw, int rpw) {
-  constexpr bool kF32 = sizeof(R) == sizeof(float);
+  constexpr bool kTable = sizeof(R) == sizeof(float) && T != kRefErfinv;
   unsigned char* icdf = nullptr;
   IcdfMasks masks;
   DyadicMasks dmasks;
-  // float32: mode 1 the shifted transform's table, mode 0 the reference
-  // transform's where the points have at most 24 digits (shl >= 8)
-  if constexpr (kF32) {
-    masks.init();
-    dmasks.init();
-    icdf = mode == 1 ? icdf_lds() : dyadic_lds();
-    if (mode == 1)
+  if constexpr (kTable) {
+    if constexpr (T == kShifted) {
+      masks.init();
+      icdf = icdf_lds();
       icdf_stage(icdf);
-    else if (shl >= 8)
+    } else {
+      dmasks.init();
+      icdf = dyadic_lds();
       dyadic_stage(icdf);
+    }
     __syncthreads();
   }
   sobol_run(v, dim, n, first, shift, dw, rpw,
             [&](int64_t i, int d, uint32_t x) {
               R z;
-              if constexpr (kF32) {
-                z = mode == 1  ? (R)icdf_shifted_f32(x, icdf, masks)
-                    : shl >= 8 ? (R)dyadic_f32(x, shl, icdf, dmasks)
-                               : sobol_ref_normal<R>(x, scale);
-              } else if (mode == 0)
-                z = sobol_ref_normal<R>(x, scale);
-              else
+              if constexpr (kTable && T == kShifted)
+                z = (R)icdf_shifted_f32(x, icdf, masks);
+              else if constexpr (kTable)
+                z = (R)dyadic_f32(x, shl, icdf, dmasks);
+              else if constexpr (T == kShifted)
                 z = sobol_shifted_normal(x, R(0));
+              else
+                z = sobol_ref_normal<R>(x, scale);
               out[i * dim + d] = z;
             });
 }
@@ -529,15 +537,18 @@ extern "C" int tqf_sobol_normals(const uint32_t* v, int32_t dim, int32_t nd,
   if (n == 0) return TQF_OK;
   const RunGrid g = run_grid(dim, n, first_index);
   if (dtype == TQF_F32) {
-    hipLaunchKernelGGL(sobol_normals_run_kernel<float>, g.grid, dim3(256), 0,
-                       (hipStream_t)stream, v, dim, std::ldexp(1.0f, -nd),
-                       32 - nd, n, first_index, shift, mode, (float*)out, g.dw,
-                       g.rpw);
+    auto kern = mode == 1 ? sobol_normals_run_kernel<float, kShifted>
+                : nd <= 24 ? sobol_normals_run_kernel<float, kRefTable>
+                          : sobol_normals_run_kernel<float, kRefErfinv>;
+    hipLaunchKernelGGL(kern, g.grid, dim3(256), 0, (hipStream_t)stream, v, dim,
+                       std::ldexp(1.0f, -nd), 32 - nd, n, first_index, shift,
+                       (float*)out, g.dw, g.rpw);
   } else {
-    hipLaunchKernelGGL(sobol_normals_run_kernel<double>, g.grid, dim3(256), 0,
-                       (hipStream_t)stream, v, dim, std::ldexp(1.0, -nd),
-                       32 - nd, n, first_index, shift, mode, (double*)out, g.dw,
-                       g.rpw);
+    auto kern = mode == 1 ? sobol_normals_run_kernel<double, kShifted>
+                          : sobol_normals_run_kernel<double, kRefErfinv>;
+    hipLaunchKernelGGL(kern, g.grid, dim3(256), 0, (hipStream_t)stream, v, dim,
+                       std::ldexp(1.0, -nd), 32 - nd, n, first_index, shift,
+                       (double*)out, g.dw, g.rpw);
   }
   return check_launch("tqf_sobol_normals");
 }
