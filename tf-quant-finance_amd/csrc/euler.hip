@@ -303,13 +303,33 @@ __device__ __forceinline__ void record(const EulerArgs<R>& a, R* lds_pay,
 
 constexpr int64_t kPairMinPaths = 1 << 16;  // see launch
 
+// Waves per SIMD asked of the compiler.  float32 Sobol kernels on coalesced
+// records or payoffs: eight, since without the bound they take 106 scalar
+// registers, which allow seven, and a launch of 2,048 workgroups (eight per
+// CU) runs its last 256 in a round of their own (2^20 paths, 100 steps, four
+// records: constant coefficients 73.5 -> 68.2 us, Hull-White 65.8 -> 60.1, QE
+// 155.5 -> 149.6, Heston 99.4 -> 98.3).  Pairs: 62 vector registers in place
+// of 66 to 70 (GBM 42.9 -> 41.2, Heston 70.4 -> 70.1), local volatility from
+// any source (180 -> 172, paired 132 -> 122).  No bound where it loses: other
+// models on plain Philox normals (QE with 365 steps 624 us, bound 641; Heston
+// 109.2, 111.5) and path-major records, whose LDS allows four workgroups a CU
+// (local volatility 148, bound 154).
+template <typename R, int MODEL, int RNG, bool kStage, bool kPair>
+constexpr int min_waves() {
+  constexpr bool kSobol = RNG == TQF_RNG_SOBOL ||
+                          RNG == TQF_RNG_SOBOL_SHIFTED ||
+                          RNG == kRngSobolDyadic;
+  return sizeof(R) == sizeof(float) && !kStage &&
+                 (kSobol || kPair || MODEL == TQF_MODEL_LOCAL_VOL)
+             ? 8
+             : 1;
+}
+
 // kPair (antithetic Philox normals, coalesced records): a thread steps path p
 // and its mirror p + n_paths / 2 with the normals drawn once.
 template <typename R, int MODEL, int RNG, bool kStage, bool kPair = false>
-// float32: eight waves per SIMD.  Without the bound the Sobol kernels take
-// 106 scalar registers, which allow seven, and a launch of 2,048 workgroups
-// (eight per CU) runs its last 256 in a round of their own.
-__global__ void __launch_bounds__(kBlock, sizeof(R) == 4 ? 8 : 1)
+__global__ void __launch_bounds__(
+    kBlock, (min_waves<R, MODEL, RNG, kStage, kPair>()))
 euler_kernel(EulerArgs<R> a) {
   constexpr int D = ModelDim<MODEL>::D;
   extern __shared__ __align__(16) unsigned char lds[];
