@@ -45,6 +45,23 @@ def test_error_path_maps_to_value_error():
                  ctypes.c_int32(0), m.ctypes.data_as(ctypes.c_void_p))
 
 
+@pytest.mark.parametrize('nd', [0, -1, 33])
+def test_exact_gbm_refuses_sobol_digits_out_of_range(nd):
+  # the float32 transform shifts by 32 - nd; checked before any launch, so
+  # also without a GPU (the addresses are not read)
+  host = np.zeros(64, np.float64)
+  addr = host.ctypes.data
+  g = _native.Gbm(dim=1, drift=addr, vol=addr, s0=addr)
+  grid = _native.Grid(dt=addr, sqrt_dt=addr, t_next=addr, slot=addr,
+                      n_steps=1, n_slots=1, init_slot=-1, n_rng_steps=1)
+  r = _native.Rng(kind=_native.RNG_SOBOL, sobol_v=addr, sobol_lo=addr,
+                  sobol_nd=nd, sobol_ndims=1)
+  with pytest.raises(ValueError, match='bad Sobol digits'):
+    _native.call('tqf_gbm_exact', ctypes.byref(g), ctypes.byref(grid),
+                 ctypes.byref(r), ctypes.c_int32(1), ctypes.c_void_p(addr),
+                 ctypes.c_int64(1), ctypes.c_int32(_native.TQF_F32), None)
+
+
 def test_native_direction_numbers_match_oracle():
   dim = 1200
   got = tsobol.direction_numbers(dim)

@@ -234,6 +234,9 @@ extern "C" int tqf_gbm_exact(const tqf_gbm* g, const tqf_grid* grid,
     TQF_REQUIRE(r->sobol_first_index >= 0 &&
                     r->sobol_first_index + n_paths <= (int64_t)0xffffffffll + 1,
                 "Sobol index range exceeds 32 bits");
+    TQF_REQUIRE(r->kind != TQF_RNG_SOBOL ||
+                    (r->sobol_nd >= 1 && r->sobol_nd <= 32),
+                "bad Sobol digits");
   }
   const hipStream_t s = (hipStream_t)stream;
   if (dtype == TQF_F32) return launch<float>(g, grid, r, out_mode, out, n_paths, s);
