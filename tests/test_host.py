@@ -62,6 +62,17 @@ def test_exact_gbm_refuses_sobol_digits_out_of_range(nd):
                  ctypes.c_int64(1), ctypes.c_int32(_native.TQF_F32), None)
 
 
+@pytest.mark.parametrize('items,blocks,steps', [(1, 1, 1), (3, 7, 16),
+                                                (128, 2, 17), (255, 64, 500)])
+def test_batch_workspace_is_what_the_kernel_carves(items, blocks, steps):
+  # item sums up to the next 256 bytes, the counter's 256, and one float per
+  # checkpoint, thread and block: the sweep keeps the variance only
+  sums = (items * 16 * 8 + 255) // 256 * 256
+  need = sums + 256 + blocks * 256 * ((steps + 15) // 16) * 4
+  got = _native.lib().tqf_batch_workspace_size(items, blocks, steps)
+  assert need <= got < need + 256
+
+
 def test_native_direction_numbers_match_oracle():
   dim = 1200
   got = tsobol.direction_numbers(dim)

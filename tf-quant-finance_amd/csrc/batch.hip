@@ -439,8 +439,8 @@ batch_finalize_kernel(const double* __restrict__ item_sums,
 extern "C" int64_t tqf_batch_workspace_size(int32_t n_items, int32_t n_blocks,
                                             int32_t max_steps) {
   const int64_t nseg = (max_steps + kSeg - 1) / kSeg;
-  return (int64_t)n_items * 2 * kStats * 8 + 256 +
-         (int64_t)n_blocks * kBlockB * nseg * 2 * 4;
+  const int64_t sums = ((int64_t)n_items * 2 * kStats * 8 + 255) & ~(int64_t)255;
+  return sums + 256 + (int64_t)n_blocks * kBlockB * nseg * 4;
 }
 
 extern "C" int tqf_batch_price(const tqf_contract* contracts,
@@ -467,7 +467,7 @@ extern "C" int tqf_batch_price(const tqf_contract* contracts,
   w += 256;
   float* ckpt = (float*)w;
   const int nseg = (max_steps + kSeg - 1) / kSeg;
-  const int64_t per_block = (int64_t)kBlockB * nseg * 2;
+  const int64_t per_block = (int64_t)kBlockB * nseg;
   hipLaunchKernelGGL(zero_counter_kernel, 1, 1, 0, s, counter);
   const int use_counter = flags & TQF_BATCH_COUNTER;
   if (flags & TQF_BATCH_TANGENT_ONLY)
