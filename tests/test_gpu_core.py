@@ -752,7 +752,7 @@ def test_heston_qe_parity(dtype, tol):
 @pytest.mark.parametrize('n', [2**16 - 2, 2**16, 2**16 + 2])
 @pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
 @pytest.mark.parametrize('name', ['gbm', 'const', 'heston_ft', 'heston_own',
-                                  'local_vol'])
+                                  'local_vol', 'heston_qe', 'hull_white'])
 def test_antithetic_rows_equal_path_major_records(name, dtype, n):
   # 2^16 paths and more step both mirrors in one thread on coalesced rows;
   # path-major records keep one path to a thread: the same bits
@@ -763,6 +763,20 @@ def test_antithetic_rows_equal_path_major_records(name, dtype, n):
     x0 = [np.log(100.)]
   elif name == 'heston_own':
     spec, x0 = ('heston', 0.0, 2.0, 0.04, 0.3, -0.7, 1.0), [np.log(100.), 0.04]
+  elif name == 'heston_qe':
+    # xi large against theta: both branches of the variance draw
+    from tqf.models import heston as heston_lib
+    model = tqf.models.HestonModel(1.2, 0.01, 0.9, -0.6, dtype=dtype)
+    npd = np.float32 if dtype == torch.float32 else np.float64
+    spec = ('heston_qe', heston_lib.qe_step_coefficients(
+        np.linspace(0.0, 1.0, 8).astype(npd), *model._params, tolerance=1e-6,
+        dtype=dtype))
+    x0 = [np.log(100.), 0.01]
+  elif name == 'hull_white':
+    model = tqf.models.hull_white.HullWhiteModel1F(
+        0.03, 0.01, lambda t: 0.02 * torch.ones_like(torch.as_tensor(t)),
+        dtype=dtype)
+    spec, x0 = ('hull_white', model._kernel_constants), [0.0]
   else:
     spec, _, x0 = _models()[name]
   all_times = np.linspace(0.0, 1.0, 8)
