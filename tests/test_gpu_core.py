@@ -773,7 +773,8 @@ def test_antithetic_rows_equal_path_major_records(name, dtype, n):
         dtype=dtype))
     x0 = [np.log(100.), 0.01]
   elif name == 'hull_white':
-    model = tqf.models.hull_white.HullWhiteModel1F(
+    from tqf.models import hull_white
+    model = hull_white.HullWhiteModel1F(
         0.03, 0.01, lambda t: 0.02 * torch.ones_like(torch.as_tensor(t)),
         dtype=dtype)
     spec, x0 = ('hull_white', model._kernel_constants), [0.0]
