@@ -72,11 +72,12 @@ constexpr int sobol_lds_words(int D) { return 2 * kSobolChunk * D; }
 // fit_icdf.py derives the table; exhaustive float32 error: 5.2e-7
 // absolute, 3.3e-7 relative for |z| >= 1e-3).
 //
-// The cubic runs on the mantissa bits placed as the float h in [1, 1.125):
-// h - 1.125 is 2^-23 times that variable, exactly, and the staged
-// coefficients carry the powers of 2^23, so every step's result is the same
-// bits as with the integer variable at one conversion less.  The upper half's
-// sign is put on the result.
+// The cubic's variable is formed by one conversion, off the chain that leads
+// to the LDS read; placed as a float's mantissa instead (one three-input
+// instruction and a subtraction of the exact offset, the same value) it made
+// launches of few waves slower: 2^16 Heston paths of 100 steps 20.2 -> 21.6
+// us, QE aside, and large ones no faster (2^20: 87.2, 87.4).  The upper
+// half's sign is put on the result.
 //
 // LDS image: segment k sits at byte ((k + 1072) & 255) * 16, which is bits
 // 20..27 of the float's bit pattern times 16 (one AND of its upper half):
@@ -100,10 +101,9 @@ __device__ __forceinline__ unsigned char* icdf_lds() {
 __device__ __forceinline__ void icdf_stage(unsigned char* lds) {
   float4* t = (float4*)lds;
   for (int e = threadIdx.x; e < kIcdfSegs; e += blockDim.x)
-    t[kIcdfSlot0 + e] =
-        make_float4(kIcdfCoef[4 * e], kIcdfCoef[4 * e + 1] * 0x1p23f,
-                    kIcdfCoef[4 * e + 2] * 0x1p46f,
-                    kIcdfCoef[4 * e + 3] * 0x1p69f);
+    t[kIcdfSlot0 + e] = make_float4(kIcdfCoef[4 * e], kIcdfCoef[4 * e + 1],
+                                    kIcdfCoef[4 * e + 2],
+                                    kIcdfCoef[4 * e + 3]);
   if (threadIdx.x == 0) t[0] = make_float4(kIcdfZero, 0.f, 0.f, 0.f);
 }
 
@@ -111,14 +111,12 @@ __device__ __forceinline__ void icdf_stage(unsigned char* lds) {
 // of three-input instructions they would halve the issue rate (see
 // PhiloxKeys).
 struct IcdfMasks {
-  uint32_t top25, low20, one, sign;
+  uint32_t top25, sign;
 
   __device__ __forceinline__ void init() {
     top25 = 0xFFFFFF80u;
-    low20 = 0x000FFFFFu;
-    one = 0x3F800000u;
     sign = 0x80000000u;
-    asm volatile("" : "+v"(top25), "+v"(low20), "+v"(one), "+v"(sign));
+    asm volatile("" : "+v"(top25), "+v"(sign));
   }
 };
 
@@ -136,9 +134,7 @@ __device__ __forceinline__ float icdf_shifted_f32(uint32_t v,
       "src0_sel:WORD_1 src1_sel:DWORD"
       : "=v"(off)
       : "v"(fi), "v"(0xFF0u));
-  // (fi & low20) | one, as a float less 1.125: [-2^-3, -2^-23]
-  const float g = __uint_as_float(__builtin_amdgcn_bitop3_b32(
-                      fi, k.low20, k.one, 0xEA)) - 1.125f;
+  const float g = (float)(int32_t)(fi | 0xFFF00000u);  // [-2^20, -1]
   const float4 c = *(const float4*)(lds + off);
   const float z = __builtin_fmaf(
       __builtin_fmaf(__builtin_fmaf(c.w, g, c.z), g, c.y), g, c.x);
