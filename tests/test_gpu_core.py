@@ -652,6 +652,33 @@ def test_euler_shifted_sobol_parity():
   _close(_np(got), want, 5e-5)
 
 
+@pytest.mark.parametrize('draws', ['sobol', 'sobol_shifted'])
+@pytest.mark.parametrize('name', ['gbm', 'heston_ft', 'local_vol'])
+def test_sobol_kernels_for_few_and_many_workgroups_agree(name, draws):
+  # float32: 7 workgroups per CU take a kernel compiled without the bound on
+  # its registers, one path more the other: the shared paths are the same bits
+  n, steps = 7 * 256 * 256, 3
+  if name == 'local_vol':
+    times, x, vols = _lv_surface()
+    spec = ('local_vol', engine.LocalVolTable(times, x[0], x[1] - x[0], vols,
+                                              0.02))
+    x0 = [np.log(100.)]
+  else:
+    spec, _, x0 = _models()[name]
+  dims = steps * len(x0)
+  rng = (engine.RngSpec.from_random_type(mvn.RandomType.SOBOL, None, 9)
+         if draws == 'sobol' else
+         engine.RngSpec('sobol_shifted', first_index=9,
+                        shift=pricing.sobol_digital_shift(dims, 7)))
+  run = lambda k: engine.run(spec, np.linspace(0.0, 1.0, steps + 1),
+                             np.array([False, True, False, True]), 2,
+                             np.asarray(x0), k, rng, torch.float32,
+                             mode='store')
+  few, many = run(n), run(n + 1)
+  assert torch.isfinite(few).all()
+  assert torch.equal(few, many[..., :n])
+
+
 # ---------------------------------------------------------- local vol
 
 def _lv_surface(nt=4, nx=9):

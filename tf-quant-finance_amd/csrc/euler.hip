@@ -302,6 +302,7 @@ __device__ __forceinline__ void record(const EulerArgs<R>& a, R* lds_pay,
 }
 
 constexpr int64_t kPairMinPaths = 1 << 16;  // see launch
+constexpr unsigned kCus = 256;  // compute units of an MI355X
 
 // Waves per SIMD asked of the compiler.  float32 Sobol kernels on coalesced
 // records or payoffs: eight, since without the bound they take 106 scalar
@@ -313,13 +314,14 @@ constexpr int64_t kPairMinPaths = 1 << 16;  // see launch
 // any source (180 -> 172, paired 132 -> 122).  No bound where it loses: other
 // models on plain Philox normals (QE with 365 steps 624 us, bound 641; Heston
 // 109.2, 111.5) and path-major records, whose LDS allows four workgroups a CU
-// (local volatility 148, bound 154).
-template <typename R, int MODEL, int RNG, bool kStage, bool kPair>
+// (local volatility 148, bound 154).  Nor where the grid leaves fewer than
+// eight waves per SIMD anyway (kFew: see launch).
+template <typename R, int MODEL, int RNG, bool kStage, bool kPair, bool kFew>
 constexpr int min_waves() {
   constexpr bool kSobol = RNG == TQF_RNG_SOBOL ||
                           RNG == TQF_RNG_SOBOL_SHIFTED ||
                           RNG == kRngSobolDyadic;
-  return sizeof(R) == sizeof(float) && !kStage &&
+  return sizeof(R) == sizeof(float) && !kStage && !kFew &&
                  (kSobol || kPair || MODEL == TQF_MODEL_LOCAL_VOL)
              ? 8
              : 1;
@@ -327,9 +329,10 @@ constexpr int min_waves() {
 
 // kPair (antithetic Philox normals, coalesced records): a thread steps path p
 // and its mirror p + n_paths / 2 with the normals drawn once.
-template <typename R, int MODEL, int RNG, bool kStage, bool kPair = false>
+template <typename R, int MODEL, int RNG, bool kStage, bool kPair = false,
+          bool kFew = false>
 __global__ void __launch_bounds__(
-    kBlock, (min_waves<R, MODEL, RNG, kStage, kPair>()))
+    kBlock, (min_waves<R, MODEL, RNG, kStage, kPair, kFew>()))
 euler_kernel(EulerArgs<R> a) {
   constexpr int D = ModelDim<MODEL>::D;
   extern __shared__ __align__(16) unsigned char lds[];
@@ -712,6 +715,30 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   TQF_PICK_RNG(TQF_MODEL_HULL_WHITE)
 #undef TQF_PICK_RNG
 #undef TQF_PICK
+  // float32 Sobol kernels with at most seven workgroups per CU: without the
+  // bound for eight waves, whose scalar spills are latency there (2^16 paths,
+  // 100 steps: local volatility 51.5 -> 47.7 us, QE 37.9 -> 36.5, GBM 17.8 ->
+  // 17.4, Heston level; at 2^18 paths level or better, at 2^19 the bound wins
+  // by 2 to 20 %)
+  if constexpr (sizeof(R) == sizeof(float)) {
+    const bool few = !stage && n_blocks <= 7 * kCus;
+#define TQF_PICK_FEW(MODEL, RNG)                                         \
+  if (few && kind == MODEL && rng_kind == RNG)                           \
+    kern = euler_kernel<R, MODEL, RNG, false, false, true>;
+#define TQF_PICK_FEW_RNG(MODEL)               \
+  TQF_PICK_FEW(MODEL, TQF_RNG_SOBOL)          \
+  TQF_PICK_FEW(MODEL, TQF_RNG_SOBOL_SHIFTED)  \
+  TQF_PICK_FEW(MODEL, kRngSobolDyadic)
+    TQF_PICK_FEW_RNG(TQF_MODEL_GBM)
+    TQF_PICK_FEW_RNG(TQF_MODEL_CONST)
+    TQF_PICK_FEW_RNG(TQF_MODEL_HESTON_FT)
+    TQF_PICK_FEW_RNG(kModelHestonOwn)
+    TQF_PICK_FEW_RNG(TQF_MODEL_LOCAL_VOL)
+    TQF_PICK_FEW_RNG(TQF_MODEL_HESTON_QE)
+    TQF_PICK_FEW_RNG(TQF_MODEL_HULL_WHITE)
+#undef TQF_PICK_FEW_RNG
+#undef TQF_PICK_FEW
+  }
 #define TQF_PICK_PAIR(MODEL) \
   if (pair && kind == MODEL) \
     kern = euler_kernel<R, MODEL, TQF_RNG_PHILOX_ANTITHETIC, false, true>;
