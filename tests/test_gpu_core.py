@@ -776,13 +776,15 @@ def test_heston_qe_parity(dtype, tol):
   _close(got[..., 1], want[..., 1], tol, scale=1e3 * np.max(want[..., 1]))
 
 
-@pytest.mark.parametrize('n', [2**16 - 2, 2**16, 2**16 + 2])
+@pytest.mark.parametrize('n', [2**16 - 2, 2**16, 2**16 + 2, 2**17, 2**17 + 2,
+                               3 * 2**16, 3 * 2**16 + 2])
 @pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
 @pytest.mark.parametrize('name', ['gbm', 'const', 'heston_ft', 'heston_own',
                                   'local_vol', 'heston_qe', 'hull_white'])
 def test_antithetic_rows_equal_path_major_records(name, dtype, n):
-  # 2^16 paths and more step both mirrors in one thread on coalesced rows;
-  # path-major records keep one path to a thread: the same bits
+  # beyond 2^16 paths (float32 2^17, local volatility and QE 3 x 2^16) both
+  # mirrors step in one thread on coalesced rows; path-major records keep one
+  # path to a thread: the same bits
   if name == 'local_vol':
     times, x, vols = _lv_surface()
     spec = ('local_vol', engine.LocalVolTable(times, x[0], x[1] - x[0], vols,

@@ -301,7 +301,6 @@ __device__ __forceinline__ void record(const EulerArgs<R>& a, R* lds_pay,
   }
 }
 
-constexpr int64_t kPairMinPaths = 1 << 16;  // see launch
 constexpr unsigned kCus = 256;  // compute units of an MI355X
 
 // Waves per SIMD asked of the compiler.  float32 Sobol kernels on coalesced
@@ -680,12 +679,24 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
   // Antithetic records on coalesced rows: both mirrors in one thread, the
   // normals (in float64 most of the step) drawn once.  float64 Brownian
   // paths, 100 records: 386 -> 264 us at 2^20 paths (839 MB), 127 -> 89 at
-  // 2^18, 76 -> 71 at 2^16; float32 139 -> 107 at 2^20.  Below 2^16 paths
-  // half the threads leave SIMDs empty and nothing is gained (69 and 71 us
-  // at 2^14).  Path-major records stage 64 consecutive paths a wave, and
+  // 2^18; float32 139 -> 107 at 2^20.  Half the threads only pay once the
+  // single ones would share their SIMDs with others.  float64: beyond one
+  // workgroup of them per CU (100 steps, four records, us single/paired: at
+  // 2^16 paths Heston 57/70, local volatility 74/84, QE 93/127, constant
+  // coefficients 34/35; at 1.5 x 2^16 89/71, 93/84, 133/128, 50/35).
+  // float32: beyond two (2^17 Heston 20.4/21.0, constant coefficients
+  // 18.3/16.5; 1.5 x 2^17 26.8/24.4, 21.3/18.9), local volatility and QE,
+  // whose own steps are long, beyond three (1.5 x 2^17 56/61, 45/52; 2^18
+  // 63/61, 54/52).  Path-major records stage 64 consecutive paths a wave, and
   // payoff sums keep their order, so both stay one path to a thread.
+  const int single_per_cu = sizeof(R) == sizeof(double) ? 1
+                            : m->kind == TQF_MODEL_LOCAL_VOL ||
+                                      m->kind == TQF_MODEL_HESTON_QE
+                                ? 3
+                                : 2;
   const bool pair = rng_kind == TQF_RNG_PHILOX_ANTITHETIC &&
-                    a.mode == TQF_OUT_STEP_MAJOR && n_paths >= kPairMinPaths;
+                    a.mode == TQF_OUT_STEP_MAJOR &&
+                    n_paths > (int64_t)single_per_cu * kCus * kBlock;
   const int64_t n_thr = pair ? n_paths / 2 : n_paths;
   const unsigned n_blocks = (unsigned)((n_thr + kBlock - 1) / kBlock);
   void (*kern)(EulerArgs<R>) = nullptr;
