@@ -728,9 +728,9 @@ int launch_typed(const tqf_model* m, const tqf_grid* g, const tqf_rng* r,
 #undef TQF_PICK
   // float32 Sobol kernels with at most seven workgroups per CU: without the
   // bound for eight waves, whose scalar spills are latency there (2^16 paths,
-  // 100 steps: local volatility 51.5 -> 47.7 us, QE 37.9 -> 36.5, GBM 17.8 ->
-  // 17.4, Heston level; at 2^18 paths level or better, at 2^19 the bound wins
-  // by 2 to 20 %)
+  // 100 steps: local volatility 51.5 -> 49.0 us, QE 37.9 -> 36.1, Heston 20.2
+  // -> 19.7; at 2^18 paths level or better, at 2^19 the bound wins by 2 to
+  // 20 %)
   if constexpr (sizeof(R) == sizeof(float)) {
     const bool few = !stage && n_blocks <= 7 * kCus;
 #define TQF_PICK_FEW(MODEL, RNG)                                         \
