@@ -525,8 +525,8 @@ def _batch(out, timed, batch_lib, pool):
                            'peak': PEAK_FP32 / 1e12, 'unit': 'TFLOP/s',
                            'frac': plan.total_flop / t / PEAK_FP32,
                            'kernel': 'batch_kernel',
-                           'flop_per_path_step': 'GBM 10, Heston 95 '
-                                                 '(tangent) / 99 (adjoint)'},
+                           'flop_per_path_step': 'GBM 6, Heston 70 '
+                                                 '(tangent) / 92 (adjoint)'},
                        'autotuned': cfg,
                        'candidates_s': {'%s/%d/%d' % (r['greeks'], r['tile'],
                                                       r['n_blocks']):

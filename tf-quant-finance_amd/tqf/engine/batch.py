@@ -31,21 +31,20 @@ GREEK_NAMES = {
 # sub/mul/max/select 1, FMA 2, sqrt/log/exp/sin/cos/div 1, integer work 0,
 # a Box-Muller normal 5 (10 per pair: 2 scale, log, mul, sqrt, sin, cos,
 # 2 mul, amortised):
-#   GBM     normal 5 + dw 1 + drift add 1 + sigma*dw FMA 2 + vega sum 1 = 10
-#   Heston, reverse mode: forward 30 (2 normals 10; max, sqrt, 2 dw;
-#           log-spot 6; variance 10) + the same 30 again when each
-#           checkpoint segment is recomputed + reverse sweep 39 (max, sqrt,
-#           2 dw 4; sqrt-bar 6; v-bar 7; rate-bar 2; kappa-bar 4; theta-bar
-#           2; xi-bar 7; rho-bar 5; v update 2) = 99
-#   Heston, tangent mode: forward 26 (2 normals 10; max, sqrt, 2 dw 4;
-#           log-spot 6; variance 6 with the shared noise term) + shared
-#           noise term 3 and 1/(2 sqrt v) 2 + five tangents x 10 (select,
-#           scale, two FMA pairs) + parameter terms 14 (kappa 3, theta 1,
-#           xi 5, rho 5) = 95
+#   GBM     normal 5 + sum 1 = 6
+#   Heston, reverse mode: forward 31 (2 normals 10; max, sqrt 2; two dw 6;
+#           shared noise term 3; log-spot 4; variance 6) + 27 again when each
+#           checkpoint segment is recomputed (no log-spot) + reverse sweep 34
+#           (max, sqrt 2; noise term 3; sqrt-bar 4; v-bar 8; kappa-bar 4;
+#           theta-bar 2; xi-bar 3; rho-bar 6; v update 2) = 92
+#   Heston, tangent mode: forward 29 (as above, the variance 4 with terms
+#           shared) + 1/(2 sqrt v) 3 and the two step factors 7 + five
+#           log-spot tangents 10 + variance tangents 21 (v0 2, kappa 5, theta
+#           3, xi 4, rho 7) = 70
 # Per-path payoff and Greek assembly (a few dozen FLOP per path) is left
 # out: at >= 50 steps it is under 1% of the total.
-FLOP_PER_PATH_STEP = {KIND_GBM: 10, KIND_HESTON: 99}
-FLOP_PER_PATH_STEP_TANGENT = {KIND_GBM: 10, KIND_HESTON: 95}
+FLOP_PER_PATH_STEP = {KIND_GBM: 6, KIND_HESTON: 92}
+FLOP_PER_PATH_STEP_TANGENT = {KIND_GBM: 6, KIND_HESTON: 70}
 GREEKS_ADJOINT, GREEKS_TANGENT = 0, 1
 _FIELDS = ['kind', 'n_steps', 'n_paths', 's0', 'strike', 'maturity', 'rate',
            'sigma', 'v0', 'kappa', 'theta', 'xi', 'rho']
