@@ -406,8 +406,8 @@ typedef struct tqf_lsm_item {
 /* Device.  tqf_lsm_price for n_items (1..16) payoffs on the same one-asset
  * paths (lsm->dim = 1, degree 0..4; lsm's payoff, strike, payoff_table,
  * n_basis and exponents are not read): basis_mask bit m says that the
- * monomial c^m is in the basis.  One launch per exercise date for all of
- * them, no host synchronisation and no host copy.  values
+ * monomial c^m is in the basis.  A pass and a solve per exercise date for
+ * all of them, no host synchronisation and no host copy.  values
  * [n_items][n_paths] (device) receives each path's value at the first
  * exercise date, before the final discount; results [n_items][2]; ranks
  * (optional) [n_items][max(n_ex - 1, 1)]. */

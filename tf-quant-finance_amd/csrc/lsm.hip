@@ -1879,8 +1879,8 @@ extern "C" int tqf_lsm_price(const tqf_lsm* l, const int32_t* ex_idx,
   const bool use_moments = moment_plan(l->dim, l->degree, n_pairs, &mp);
   const int ndense = dense_size(l->dim, l->degree, K);
   LsmArgs a = make_args(&l2, ex_idx[n_ex - 1]);
-  // one asset up to degree kChainMaxDeg: one launch per date (its state fits
-  // the Gram partials' buffer up to some thousands of dates)
+  // one asset up to degree kChainMaxDeg: a pass and a solve per date (its
+  // state fits the Gram partials' buffer up to some thousands of dates)
   if (l->dim == 1 && l->degree <= kChainMaxDeg &&
       chain_workspace(n, 1, n_ex) <=
           (int64_t)256 * n_pairs * kTile * kTile * 8) {

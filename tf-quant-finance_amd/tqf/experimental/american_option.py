@@ -14,10 +14,12 @@ Here the Brownian paths W(t) come from the fused kernel's constant-
 coefficient model with the engine's antithetic Philox stream (the
 reference's STATELESS_ANTITHETIC), and the options are regressed together
 in the FP64 one-asset LSM kernels (tqf_lsm_price_shared: basis on ln S,
-payoff on S), one launch per exercise date.  ln(S / S0) is an affine map of
-W(t) per option and date, which the standardised basis does not see, so the
-kernels read W itself and no option has paths of its own.  A user basis_fn falls back to the torch LSM with the same
-log-path / payoff split.
+payoff on S), a pass and a solve per exercise date.  ln(S / S0) is an affine
+map of W(t) per option and date, which the standardised basis does not see,
+so the kernels read W itself and no option has paths of its own.  Degrees the
+shared kernels do not take run option by option on up to four side streams.
+A user basis_fn falls back to the torch LSM with the same log-path / payoff
+split.
 """
 import numpy as np
 import torch
